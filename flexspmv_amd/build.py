@@ -53,7 +53,7 @@ def _csrc_digest() -> str:
     h = hashlib.sha1()
     for root in (CSRC_DIR, INCLUDE_DIR):
         for fn in sorted(os.listdir(root)):
-            if fn.endswith((".hpp", ".h")) and fn != "flexspmv_formats.h":
+            if fn.endswith((".hpp", ".h")) and fn not in ("flexspmv_formats.h", "flexspmv_vectors.h"):
                 with open(os.path.join(root, fn), "rb") as f:
                     h.update(fn.encode())
                     h.update(f.read())
@@ -132,40 +132,50 @@ def compile_many(graphs: Iterable[FusedGraphIR], jobs: int = 8, force: bool = Fa
 
 
 # ---------------------------------------------------------------------------------------------
-# the edge-list preparation library (one per package, not per sub-graph)
+# the libraries there is one of per package, not per sub-graph: edge-list preparation, vector updates
 # ---------------------------------------------------------------------------------------------
 FORMATS_SOURCE = os.path.join(CSRC_DIR, "flex_formats.hip")
 FORMATS_LIBRARY = os.path.join(GENERATED_DIR, "libflexspmv_formats.so")
+VECTORS_SOURCE = os.path.join(CSRC_DIR, "flex_vectors.hip")
+VECTORS_LIBRARY = os.path.join(GENERATED_DIR, "libflexspmv_vectors.so")
+_PARTS = {FORMATS_LIBRARY: (FORMATS_SOURCE, os.path.join(INCLUDE_DIR, "flexspmv_formats.h")),
+          VECTORS_LIBRARY: (VECTORS_SOURCE, os.path.join(INCLUDE_DIR, "flexspmv_vectors.h"),
+                            os.path.join(CSRC_DIR, "flex_wave.hpp"))}
 
 
-def _formats_stamp() -> str:
+def _parts_stamp(library: str) -> str:
     h = hashlib.sha1()
-    for path in (FORMATS_SOURCE, os.path.join(INCLUDE_DIR, "flexspmv_formats.h")):
+    for path in _PARTS[library]:
         with open(path, "rb") as f:
             h.update(f.read())
     return h.hexdigest() + ":" + " ".join(HIPCC_FLAGS)
 
 
-def formats_is_current() -> bool:
-    stamp = _stamp_path(FORMATS_LIBRARY)
-    if not (os.path.exists(FORMATS_LIBRARY) and os.path.exists(stamp)):
-        return False
-    with open(stamp) as f:
-        return f.read() == _formats_stamp()
+def _compile_parts(library: str, force: bool) -> str:
+    stamp = _stamp_path(library)
+    if not force and os.path.exists(library) and os.path.exists(stamp):
+        with open(stamp) as f:
+            if f.read() == _parts_stamp(library):
+                return library
+    os.makedirs(GENERATED_DIR, exist_ok=True)
+    source = _PARTS[library][0]
+    cmd = [hipcc_path(), *HIPCC_FLAGS, f"-I{CSRC_DIR}", f"-I{INCLUDE_DIR}", source, "-o", library]
+    proc = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    if proc.returncode != 0:
+        raise BuildError(f"hipcc failed for {os.path.basename(source)}:\n{' '.join(cmd)}\n{proc.stdout}")
+    with open(stamp, "w") as f:
+        f.write(_parts_stamp(library))
+    return library
 
 
 def compile_formats(force: bool = False) -> str:
     """Compile csrc/flex_formats.hip into _generated/libflexspmv_formats.so; returns its path."""
-    if not force and formats_is_current():
-        return FORMATS_LIBRARY
-    os.makedirs(GENERATED_DIR, exist_ok=True)
-    cmd = [hipcc_path(), *HIPCC_FLAGS, f"-I{INCLUDE_DIR}", FORMATS_SOURCE, "-o", FORMATS_LIBRARY]
-    proc = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
-    if proc.returncode != 0:
-        raise BuildError(f"hipcc failed for the formats library:\n{' '.join(cmd)}\n{proc.stdout}")
-    with open(_stamp_path(FORMATS_LIBRARY), "w") as f:
-        f.write(_formats_stamp())
-    return FORMATS_LIBRARY
+    return _compile_parts(FORMATS_LIBRARY, force)
+
+
+def compile_vectors(force: bool = False) -> str:
+    """Compile csrc/flex_vectors.hip into _generated/libflexspmv_vectors.so; returns its path."""
+    return _compile_parts(VECTORS_LIBRARY, force)
 
 
 # ---------------------------------------------------------------------------------------------

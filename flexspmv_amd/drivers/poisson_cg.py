@@ -8,6 +8,7 @@ from typing import Callable, Tuple
 
 import torch
 
+from .. import vectors
 from .. import workloads as W
 from ..binding import load_named
 
@@ -29,22 +30,28 @@ def fused_operator(n: int, device="cuda", dtype=torch.float64) -> Tuple[Callable
 
 
 def conjugate_gradients(apply: Callable, b: torch.Tensor, tol: float = 1e-10, maxiter: int = 1000):
-    """Solve ``A x = b``; returns (x, iterations, relative residual).  All scalars stay on the device."""
+    """Solve ``A x = b``; returns (x, iterations, relative residual).  All scalars stay on the device.
+
+    On the GPU the vector updates of an iteration are two kernels (``flexspmv_amd.vectors``); elsewhere, and where
+    ``apply`` returns something those kernels do not take, torch's operators."""
     x = torch.zeros_like(b)
     r = b.clone()
     p = r.clone()
     rr = torch.dot(r, r)
     stop = (tol * tol) * rr
+    updates = vectors.ConjugateGradientUpdates(b) if vectors.supports(b) else None
     it = 0
     for it in range(1, maxiter + 1):
         ap, pap = apply(p)
-        alpha = rr / pap[0]
-        x.add_(p * alpha)
-        r.sub_(ap * alpha)
-        rr_new = torch.dot(r, r)
-        if it % 8 == 0 and bool(rr_new <= stop):      # one host synchronisation every 8 iterations
-            rr = rr_new
-            break
-        p = r + p * (rr_new / rr)
+        if updates is not None and updates.takes(ap, pap):
+            p, rr_new = updates.step(x, r, p, ap, rr, pap)
+        else:
+            alpha = rr / pap[0]
+            x.add_(p * alpha)
+            r.sub_(ap * alpha)
+            rr_new = torch.dot(r, r)
+            p = r + p * (rr_new / rr)
         rr = rr_new
+        if it % 8 == 0 and bool(rr <= stop):      # one host synchronisation every 8 iterations
+            break
     return x, it, float(torch.sqrt(rr / torch.dot(b, b)))

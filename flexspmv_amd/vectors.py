@@ -1,0 +1,85 @@
+"""Host side of the vector update library (``include/flexspmv_vectors.h``): the two kernels of a
+conjugate-gradient iteration that are not the fused ``y = A p``, ``p . y`` launch, on torch's device memory and
+current stream."""
+from __future__ import annotations
+
+import ctypes
+import os
+from typing import Optional, Tuple
+
+from . import build as _build
+
+ABI_VERSION = 1
+MAX_PARTIALS = 2048          # FLEXSPMV_CG_MAX_PARTIALS
+EXPORTED_SYMBOLS = ("flexspmv_cg_step", "flexspmv_cg_direction", "flexspmv_vectors_last_error",
+                    "flexspmv_vectors_abi_version")
+
+_lib: Optional[ctypes.CDLL] = None
+
+
+def load_library(path: Optional[str] = None) -> ctypes.CDLL:
+    """dlopen the vector update library and type its entry points."""
+    path = path or _build.VECTORS_LIBRARY
+    if not os.path.exists(path):
+        raise RuntimeError(f"FlexSpmv vector update library {path} is not built (run __graft_entry__.build())")
+    import torch  # noqa: F401  (torch's HIP runtime has to be the one in the process)
+    lib = ctypes.CDLL(path, mode=ctypes.RTLD_LOCAL)
+    vp, i64, i32 = ctypes.c_void_p, ctypes.c_int64, ctypes.c_int
+    lib.flexspmv_cg_step.argtypes = [vp, vp, vp, vp, vp, vp, i64, i32, vp, vp]
+    lib.flexspmv_cg_step.restype = ctypes.c_int
+    lib.flexspmv_cg_direction.argtypes = [vp, vp, vp, vp, vp, vp, i64, i32, vp]
+    lib.flexspmv_cg_direction.restype = ctypes.c_int
+    lib.flexspmv_vectors_last_error.argtypes = []
+    lib.flexspmv_vectors_last_error.restype = ctypes.c_char_p
+    lib.flexspmv_vectors_abi_version.argtypes = []
+    lib.flexspmv_vectors_abi_version.restype = ctypes.c_int
+    if lib.flexspmv_vectors_abi_version() != ABI_VERSION:
+        raise RuntimeError(f"{path} was built against vectors ABI {lib.flexspmv_vectors_abi_version()}, "
+                           f"this package expects {ABI_VERSION}; rebuild it")
+    return lib
+
+
+def library() -> ctypes.CDLL:
+    global _lib
+    if _lib is None:
+        _lib = load_library()
+    return _lib
+
+
+def supports(b) -> bool:
+    """Vectors the kernels take: non-empty contiguous float32 / float64 on the GPU."""
+    import torch
+    return b.is_cuda and b.dim() == 1 and b.numel() > 0 and b.is_contiguous() \
+        and b.dtype in (torch.float32, torch.float64) and not b.requires_grad
+
+
+class ConjugateGradientUpdates:
+    """``x += alpha p, r -= alpha A p, p = r + beta p`` of one solve, with its scratch."""
+
+    def __init__(self, b) -> None:
+        import torch
+        self._n, self._dtype, self._device = b.numel(), b.dtype, b.device
+        self._bytes = b.element_size()
+        self._partials = torch.empty(MAX_PARTIALS, dtype=b.dtype, device=b.device)
+        self._lib = library()
+
+    def takes(self, ap, pap) -> bool:
+        return (ap.dtype == self._dtype and ap.device == self._device and ap.numel() == self._n and ap.is_contiguous()
+                and pap.dtype == self._dtype and pap.device == self._device and pap.numel() > 0)
+
+    def step(self, x, r, p, ap, rr, pap) -> Tuple["torch.Tensor", "torch.Tensor"]:
+        """Updates ``x`` and ``r`` in place; returns the next direction and the new ``r . r`` (0-dim, on the device)."""
+        import torch
+        lib, n = self._lib, self._n
+        p_next = torch.empty_like(p)
+        rr_new = torch.empty_like(rr)
+        with torch.cuda.device(self._device):
+            stream = torch.cuda.current_stream().cuda_stream
+            rc = lib.flexspmv_cg_step(x.data_ptr(), r.data_ptr(), p.data_ptr(), ap.data_ptr(), rr.data_ptr(),
+                                      pap.data_ptr(), n, self._bytes, self._partials.data_ptr(), stream)
+            if rc == 0:
+                rc = lib.flexspmv_cg_direction(p_next.data_ptr(), p.data_ptr(), r.data_ptr(), rr.data_ptr(),
+                                               rr_new.data_ptr(), self._partials.data_ptr(), n, self._bytes, stream)
+        if rc != 0:
+            raise RuntimeError(f"flexspmv vector update failed ({rc}): {lib.flexspmv_vectors_last_error().decode()}")
+        return p_next, rr_new

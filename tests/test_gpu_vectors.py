@@ -1,0 +1,49 @@
+"""The vector update kernels of a conjugate-gradient iteration against the same updates in float64 numpy."""
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+
+pytestmark = pytest.mark.gpu
+
+# one value; around a 16-byte word; around a block's share (2 words per thread) in both types; two rounds of the
+# largest grid (2048 blocks) and a remainder
+SIZES = (1, 2, 3, 5, 255, 1023, 1024, 1025, 2049, 70_001, 2048 * 1024, 2048 * 1024 * 2 + 1027)
+
+
+@pytest.mark.parametrize("dtype", ["float32", "float64"])
+@pytest.mark.parametrize("offset", [0, 1])          # arrays on and off 16-byte boundaries
+@pytest.mark.parametrize("n", SIZES)
+def test_updates_against_numpy(n, offset, dtype):
+    from flexspmv_amd.vectors import ConjugateGradientUpdates
+    print(f"case cg updates {n} {offset} {dtype}", flush=True)
+    rng = np.random.default_rng(n)
+    host = {k: rng.uniform(-1.0, 1.0, n).astype(dtype) for k in ("x", "r", "p", "ap")}
+    rr, pap = (rng.uniform(1.0, 2.0, 1).astype(dtype) for _ in range(2))
+
+    def on_gpu(a):
+        whole = torch.empty(n + offset, dtype=getattr(torch, dtype), device="cuda")
+        whole[offset:] = torch.from_numpy(a).cuda()
+        return whole[offset:]
+
+    g = {k: on_gpu(v) for k, v in host.items()}
+    updates = ConjugateGradientUpdates(g["x"])
+    p_next, rr_new = updates.step(g["x"], g["r"], g["p"], g["ap"], torch.from_numpy(rr).cuda()[0],
+                                   torch.from_numpy(pap).cuda())
+    eps = np.finfo(dtype).eps
+    h = {k: v.astype(np.float64) for k, v in host.items()}
+    alpha = float(rr[0]) / float(pap[0])
+    x, r = h["x"] + alpha * h["p"], h["r"] - alpha * h["ap"]
+    # alpha, the product and the sum are rounded once each
+    bound = 2 * eps * (np.abs(h["x"]) + 2 * np.abs(alpha * h["p"]))
+    assert np.all(np.abs(g["x"].cpu().numpy() - x) <= bound)
+    bound_r = 2 * eps * (np.abs(h["r"]) + 2 * np.abs(alpha * h["ap"]))
+    assert np.all(np.abs(g["r"].cpu().numpy() - r) <= bound_r)
+    # the sum of squares of the rounded r: a thread's chain, the wavefront's six steps, the partials' chains
+    mine = g["r"].cpu().numpy().astype(np.float64)
+    chain = n / (2048 * 256) + 8 + 2 * 10 + 8
+    want = float(np.dot(mine, mine))
+    assert abs(float(rr_new) - want) <= chain * eps * want
+    beta = float(rr_new) / float(rr[0])
+    want_p = mine + beta * h["p"]
+    assert np.all(np.abs(p_next.cpu().numpy() - want_p) <= 2 * eps * (np.abs(mine) + 2 * np.abs(beta * h["p"])))
