@@ -98,6 +98,27 @@ def load_library(path: str) -> ctypes.CDLL:
     return lib
 
 
+_host: Any = None
+
+
+def host_module():
+    """The native launch path (csrc/host_launch.cpp), loaded once."""
+    global _host
+    if _host is None:
+        import importlib.machinery
+        import importlib.util
+
+        import torch  # noqa: F401  (the extension resolves against the torch that is in the process)
+        path = _build.HOST_LIBRARY
+        if not os.path.exists(path):
+            raise RuntimeError(f"{path} is not built (run __graft_entry__.build())")
+        loader = importlib.machinery.ExtensionFileLoader("flexspmv_host", path)
+        module = importlib.util.module_from_spec(importlib.util.spec_from_file_location("flexspmv_host", path, loader=loader))
+        loader.exec_module(module)
+        _host = module
+    return _host
+
+
 def variant_of(signature: Dict[str, Any]) -> str:
     """What makes a library a measurement variant - its tuning switches and tile-shape override as text -
     or "" for a product library."""
@@ -183,10 +204,25 @@ class HipExtension:
         self._out_specs = [(o["kind"], int(o["dim"])) for o in self._outputs]
         self._ws_bytes: Dict[Any, int] = {}
         self._tls = threading.local()
+        self._native = self._native_launch()
 
     # -- helpers -------------------------------------------------------------------------
     def param_names(self) -> List[str]:
         return list(self._param_names)
+
+    def _native_launch(self):
+        """``launch(self, args)`` of csrc/host_launch.cpp for this library."""
+        where = {n: i for i, n in enumerate(self._param_names)}
+        lead = {"sum": 0, "reducer": 1}
+        dtypes = sum(1 << DTYPE_CODES[d] for d in self._dtypes if d != "int64" or self.signature["allow_int64"])
+        address = [ctypes.cast(f, ctypes.c_void_p).value for f in
+                   (self._lib.flexspmv_launch, self._lib.flexspmv_workspace_bytes, self._lib.flexspmv_last_error)]
+        return host_module().Launcher(
+            *address, len(self._param_names), where[self._dispatch_name], where["row_end_offsets"], where["num_rows"],
+            where["num_cols"], dtypes, self._has_reducer,
+            tuple((where[n], self._dims[n], n in self._streamed, n in self._row_indexed) for n in self._value_names),
+            tuple(where[n] for n in self._index_names),
+            tuple((lead.get(kind, 2), dim) for kind, dim in self._out_specs), self._workspace, self._last_used).launch
 
     def _bind(self, args: Sequence[Any], kwargs: Dict[str, Any]) -> Dict[str, Any]:
         names = self._param_names
@@ -311,6 +347,15 @@ class HipExtension:
         return rep
 
     def merged_spmv_launch(self, *args, **kwargs):
+        # A library's first launch, and what the native path does not take (it says so before it has done anything:
+        # keywords, a failed check, a stream capture, timing and debugging options), go through Python.
+        if self._launch_count and not kwargs:
+            outs = self._native(self, args)
+            if outs is not NotImplemented:
+                return outs
+        return self._launch_checked(args, kwargs)
+
+    def _launch_checked(self, args, kwargs):
         import torch
         if not kwargs and not self.verify_row_aligned:
             rep = self._same_arguments(args)

@@ -151,19 +151,28 @@ def _parts_stamp(library: str) -> str:
     return h.hexdigest() + ":" + " ".join(HIPCC_FLAGS)
 
 
-def _compile_parts(library: str, force: bool) -> str:
+def _parts_current(library: str) -> bool:
     stamp = _stamp_path(library)
-    if not force and os.path.exists(library) and os.path.exists(stamp):
-        with open(stamp) as f:
-            if f.read() == _parts_stamp(library):
-                return library
+    if not (os.path.exists(library) and os.path.exists(stamp)):
+        return False
+    with open(stamp) as f:
+        return f.read() == _parts_stamp(library)
+
+
+def formats_is_current() -> bool:
+    return _parts_current(FORMATS_LIBRARY)
+
+
+def _compile_parts(library: str, force: bool) -> str:
+    if not force and _parts_current(library):
+        return library
     os.makedirs(GENERATED_DIR, exist_ok=True)
     source = _PARTS[library][0]
     cmd = [hipcc_path(), *HIPCC_FLAGS, f"-I{CSRC_DIR}", f"-I{INCLUDE_DIR}", source, "-o", library]
     proc = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
     if proc.returncode != 0:
         raise BuildError(f"hipcc failed for {os.path.basename(source)}:\n{' '.join(cmd)}\n{proc.stdout}")
-    with open(stamp, "w") as f:
+    with open(_stamp_path(library), "w") as f:
         f.write(_parts_stamp(library))
     return library
 
@@ -176,6 +185,45 @@ def compile_formats(force: bool = False) -> str:
 def compile_vectors(force: bool = False) -> str:
     """Compile csrc/flex_vectors.hip into _generated/libflexspmv_vectors.so; returns its path."""
     return _compile_parts(VECTORS_LIBRARY, force)
+
+
+# ---------------------------------------------------------------------------------------------
+# the native launch path (a CPython extension against torch's headers; host code only)
+# ---------------------------------------------------------------------------------------------
+HOST_SOURCE = os.path.join(CSRC_DIR, "host_launch.cpp")
+HOST_LIBRARY = os.path.join(GENERATED_DIR, "flexspmv_host.so")
+
+
+def compile_host(force: bool = False) -> str:
+    """Compile csrc/host_launch.cpp into _generated/flexspmv_host.so; returns its path."""
+    import sysconfig
+
+    import torch
+    root = os.path.dirname(torch.__file__)
+    flags = ["-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM",
+             f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+             "-isystem", os.path.join(root, "include"),
+             "-isystem", os.path.join(root, "include", "torch", "csrc", "api", "include"),
+             "-isystem", os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "include"),
+             "-isystem", sysconfig.get_paths()["include"], f"-I{INCLUDE_DIR}"]
+    libs = ["-L" + os.path.join(root, "lib"), "-ltorch_python", "-ltorch", "-ltorch_cpu", "-ltorch_hip", "-lc10", "-lc10_hip"]
+    h = hashlib.sha1()
+    for path in (HOST_SOURCE, os.path.join(INCLUDE_DIR, "flexspmv.h")):
+        with open(path, "rb") as f:
+            h.update(f.read())
+    stamp = ":".join([h.hexdigest(), torch.__version__, " ".join(flags)])
+    if not force and os.path.exists(HOST_LIBRARY) and os.path.exists(_stamp_path(HOST_LIBRARY)):
+        with open(_stamp_path(HOST_LIBRARY)) as f:
+            if f.read() == stamp:
+                return HOST_LIBRARY
+    os.makedirs(GENERATED_DIR, exist_ok=True)
+    cmd = [os.environ.get("CXX", "g++"), *flags, HOST_SOURCE, *libs, "-o", HOST_LIBRARY]
+    proc = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    if proc.returncode != 0:
+        raise BuildError(f"the native launch path did not compile:\n{' '.join(cmd)}\n{proc.stdout}")
+    with open(_stamp_path(HOST_LIBRARY), "w") as f:
+        f.write(stamp)
+    return HOST_LIBRARY
 
 
 # ---------------------------------------------------------------------------------------------

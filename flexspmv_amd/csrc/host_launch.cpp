@@ -1,0 +1,341 @@
+// Host side of a launch of a generated library, as a CPython extension: argument checks, outputs, scratch look-up and
+// the C call (flexspmv.h) without a line of Python in between.
+//
+// A launch of a few thousand rows runs on the GPU for 5 to 7 us.  Checked, allocated and issued from Python a pass took
+// 17.0 us on a 256 x 256 Laplacian (18.7 on a 61 x 47 x 83 stencil with a dot product, a step of the shallow-water
+// model on 45 000 cells 530), from here 8.1 (9.5, 242): the GPU's own time and little more.  The checks are those of
+// HipExtension._launch_checked (flexspmv_amd/binding.py), which stays the place that words the errors: whatever this
+// function does not take - a failed check, a keyword, a launch under a stream capture or on another device, a debugging
+// option - it hands back by returning NotImplemented, before anything has happened, and the Python path does it.
+#define PY_SSIZE_T_CLEAN
+#include <Python.h>
+
+#include <ATen/core/Tensor.h>
+#include <ATen/hip/EmptyTensor.h>
+#include <c10/hip/HIPFunctions.h>
+#include <c10/hip/HIPStream.h>
+#include <hip/hip_runtime_api.h>
+#include <torch/csrc/Device.h>
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/utils/object_ptr.h>
+
+#include <memory>
+#include <vector>
+
+#include "flexspmv.h"
+
+namespace {
+
+using LaunchFn = int (*)(const flexspmv_launch_args*);
+using WorkspaceFn = size_t (*)(int32_t, int64_t, int64_t);
+using ErrorFn = const char* (*)();
+
+struct ValueArg {
+  int pos;            // position in the call's arguments
+  int64_t dim;        // values per item
+  bool streamed;      // one item per edge
+  bool row_indexed;   // one item per row
+};
+struct Output {
+  int lead;           // 0: one item, 1: an item per row, 2: an item per edge
+  int64_t dim;
+};
+
+struct Plan {
+  LaunchFn launch;
+  WorkspaceFn workspace_bytes;
+  ErrorFn last_error;
+  int num_args, dispatch_pos, ro_pos, rows_pos, cols_pos;
+  int dtype_mask;     // bit per FLEXSPMV_F32 / F64 / I64
+  bool has_reducer;
+  std::vector<ValueArg> values;
+  std::vector<int> indices;
+  std::vector<Output> outputs;
+};
+
+struct Launcher {
+  PyObject_HEAD
+  Plan* plan;
+  PyObject* workspace;   // HipExtension._workspace: (device index, stream, row pointer address) -> scratch tensor
+  PyObject* last_used;   // HipExtension._last_used
+};
+
+PyObject *s_time_kernel, *s_extra_flags, *s_reuse_tiles, *s_verify, *s_launch_count;
+
+PyObject* refuse() { Py_RETURN_NOTIMPLEMENTED; }
+
+// A tensor argument the kernels can take as it is, or nullptr.
+inline const at::Tensor* usable(PyObject* o) {
+  if (!THPVariable_Check(o)) return nullptr;
+  const at::Tensor& t = THPVariable_Unpack(o);
+  return t.is_cuda() && t.is_contiguous() ? &t : nullptr;
+}
+
+// Is the option set?  (-1: an error is pending)
+inline int option_set(PyObject* ext, PyObject* name) {
+  PyObject* v = PyObject_GetAttr(ext, name);
+  if (v == nullptr) return -1;
+  const int on = v == Py_False ? 0 : PyObject_IsTrue(v);
+  Py_DECREF(v);
+  return on;
+}
+
+// The scratch of this launch; a new reference, or nullptr with an error set.
+PyObject* scratch_of(Launcher* self, PyObject* ext, const c10::Device& device, long long stream, long long row_ptr,
+                     size_t bytes) {
+  PyObject* key = Py_BuildValue("(iLL)", (int)device.index(), stream, row_ptr);
+  if (key == nullptr) return nullptr;
+  PyObject* found = PyDict_GetItemWithError(self->workspace, key);
+  if (found != nullptr && THPVariable_Check(found) && (size_t)THPVariable_Unpack(found).numel() >= bytes) {
+    Py_INCREF(found);
+    PyObject* count = PyObject_GetAttr(ext, s_launch_count);
+    PyObject* next = count != nullptr ? PyLong_FromLongLong(PyLong_AsLongLong(count) + 1) : nullptr;
+    Py_XDECREF(count);
+    const bool counted = next != nullptr && PyObject_SetAttr(ext, s_launch_count, next) == 0 &&
+                         PyDict_SetItem(self->last_used, key, next) == 0;
+    Py_XDECREF(next);
+    Py_DECREF(key);
+    if (!counted) {
+      Py_DECREF(found);
+      return nullptr;
+    }
+    return found;
+  }
+  Py_DECREF(key);
+  if (PyErr_Occurred()) return nullptr;
+  PyObject* dev = THPDevice_New(device);
+  if (dev == nullptr) return nullptr;
+  PyObject* made = PyObject_CallMethod(ext, "_scratch", "OiLnL", dev, (int)device.index(), stream, (Py_ssize_t)bytes, row_ptr);
+  Py_DECREF(dev);
+  if (made != nullptr && !THPVariable_Check(made)) {
+    Py_DECREF(made);
+    PyErr_SetString(PyExc_TypeError, "_scratch() must return a tensor");
+    return nullptr;
+  }
+  return made;
+}
+
+constexpr int MAX_POINTERS = 64;  // of one kind; a library with more goes through Python
+
+// launch(extension, arguments) -> tuple of outputs | None | NotImplemented
+PyObject* launcher_launch(PyObject* self_obj, PyObject* const* call, Py_ssize_t ncall) {
+  HANDLE_TH_ERRORS
+  Launcher* self = reinterpret_cast<Launcher*>(self_obj);
+  const Plan& plan = *self->plan;
+  if (ncall != 2 || !PyTuple_Check(call[1])) {
+    PyErr_SetString(PyExc_TypeError, "launch(extension, arguments)");
+    return nullptr;
+  }
+  PyObject *ext = call[0], *args = call[1];
+  if (PyTuple_GET_SIZE(args) != plan.num_args) return refuse();
+  for (PyObject* name : {s_time_kernel, s_extra_flags, s_reuse_tiles, s_verify}) {
+    const int on = option_set(ext, name);
+    if (on != 0) return on < 0 ? nullptr : refuse();
+  }
+  PyObject *rows_obj = PyTuple_GET_ITEM(args, plan.rows_pos), *cols_obj = PyTuple_GET_ITEM(args, plan.cols_pos);
+  if (!PyLong_CheckExact(rows_obj) || !PyLong_CheckExact(cols_obj)) return refuse();
+  int overflow_rows = 0, overflow_cols = 0;
+  const int64_t num_rows = PyLong_AsLongLongAndOverflow(rows_obj, &overflow_rows);
+  const int64_t num_cols = PyLong_AsLongLongAndOverflow(cols_obj, &overflow_cols);
+  if (overflow_rows != 0 || overflow_cols != 0 || num_rows < 0) return refuse();
+
+  const at::Tensor* dispatch = usable(PyTuple_GET_ITEM(args, plan.dispatch_pos));
+  const at::Tensor* ro = usable(PyTuple_GET_ITEM(args, plan.ro_pos));
+  if (dispatch == nullptr || ro == nullptr || ro->scalar_type() != at::kInt) return refuse();
+  const at::ScalarType dtype = dispatch->scalar_type();
+  int code;
+  switch (dtype) {
+    case at::kFloat: code = FLEXSPMV_F32; break;
+    case at::kDouble: code = FLEXSPMV_F64; break;
+    case at::kLong: code = FLEXSPMV_I64; break;
+    default: return refuse();
+  }
+  if (((plan.dtype_mask >> code) & 1) == 0) return refuse();
+  const c10::Device device = dispatch->device();
+  if (device.index() != c10::hip::current_device()) return refuse();
+
+  const void* index_ptrs[MAX_POINTERS];
+  void *value_ptrs[MAX_POINTERS], *output_ptrs[MAX_POINTERS];
+  int64_t ne = num_cols;
+  for (size_t i = 0; i < plan.indices.size(); ++i) {
+    const at::Tensor* t = usable(PyTuple_GET_ITEM(args, plan.indices[i]));
+    if (t == nullptr || t->scalar_type() != at::kInt) return refuse();
+    if (i == 0) ne = t->numel();
+    if (t->numel() != ne) return refuse();
+    index_ptrs[i] = t->data_ptr();
+  }
+  if (ne <= 0) return refuse();
+  for (size_t i = 0; i < plan.values.size(); ++i) {
+    const ValueArg& v = plan.values[i];
+    const at::Tensor* t = usable(PyTuple_GET_ITEM(args, v.pos));
+    if (t == nullptr || t->scalar_type() != dtype) return refuse();
+    const int64_t count = t->numel();
+    if (count % v.dim != 0 || (v.streamed && count < ne * v.dim)) return refuse();
+    if (v.row_indexed && count < num_rows * v.dim && num_rows + ne < ((int64_t)1 << 31)) return refuse();
+    value_ptrs[i] = t->data_ptr();
+  }
+  if (plan.has_reducer && ro->numel() != num_rows + 1) return refuse();
+
+  const hipStream_t stream = c10::hip::getCurrentHIPStream(device.index()).stream();
+  hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(stream, &capturing) != hipSuccess || capturing != hipStreamCaptureStatusNone) {
+    (void)hipGetLastError();
+    return refuse();
+  }
+  const size_t bytes = plan.workspace_bytes(code, num_rows, ne);
+  PyObject* scratch = scratch_of(self, ext, device, (long long)(intptr_t)stream,
+                                 plan.has_reducer ? (long long)(intptr_t)ro->data_ptr() : 0, bytes);
+  if (scratch == nullptr) return nullptr;
+  THPObjectPtr scratch_owner(scratch);
+  const at::Tensor& ws = THPVariable_Unpack(scratch);
+
+  const Py_ssize_t num_outputs = (Py_ssize_t)plan.outputs.size();
+  THPObjectPtr result(num_outputs > 0 ? PyTuple_New(num_outputs) : nullptr);
+  if (num_outputs > 0 && !result) return nullptr;
+  for (Py_ssize_t i = 0; i < num_outputs; ++i) {
+    const Output& o = plan.outputs[i];
+    const int64_t lead = o.lead == 1 ? num_rows : ne;
+    const int64_t sizes[2] = {o.lead == 0 ? o.dim : lead, o.dim};
+    const int64_t rank = o.lead == 0 || o.dim == 1 ? 1 : 2;
+    at::Tensor out(at::detail::empty_cuda(c10::IntArrayRef(sizes, rank), dtype, device, std::nullopt));
+    output_ptrs[i] = out.data_ptr();
+    PyObject* wrapped = THPVariable_Wrap(std::move(out));
+    if (wrapped == nullptr) return nullptr;
+    PyTuple_SET_ITEM(result.get(), i, wrapped);
+  }
+
+  flexspmv_launch_args la{};
+  la.struct_size = sizeof(la);
+  la.dtype = code;
+  la.value_inputs = value_ptrs;
+  la.num_value_inputs = (int32_t)plan.values.size();
+  la.index_inputs = reinterpret_cast<const int32_t* const*>(index_ptrs);
+  la.num_index_inputs = (int32_t)plan.indices.size();
+  la.outputs = output_ptrs;
+  la.num_outputs = (int32_t)num_outputs;
+  la.row_end_offsets = static_cast<const int32_t*>(ro->data_ptr());
+  la.num_rows = num_rows;
+  la.num_cols = num_cols;
+  la.ne = ne;
+  la.workspace = ws.data_ptr();
+  la.workspace_bytes = (size_t)ws.numel();
+  la.stream = stream;
+  int rc;
+  {
+    pybind11::gil_scoped_release no_gil;
+    rc = plan.launch(&la);
+  }
+  if (rc != FLEXSPMV_OK) {
+    PyErr_Format(PyExc_RuntimeError, "merged_spmv_launch failed (%d): %s", rc, plan.last_error());
+    return nullptr;
+  }
+  if (num_outputs == 0) Py_RETURN_NONE;
+  return result.release();
+  END_HANDLE_TH_ERRORS
+}
+
+// Launcher(launch, workspace_bytes, last_error, num_args, dispatch_pos, ro_pos, rows_pos, cols_pos, dtype_mask,
+//          has_reducer, ((pos, dim, streamed, row_indexed), ...), (pos, ...), ((lead, dim), ...), workspace, last_used)
+PyObject* launcher_new(PyTypeObject* type, PyObject* args, PyObject*) {
+  unsigned long long launch, workspace_bytes, last_error;
+  int num_args, dispatch_pos, ro_pos, rows_pos, cols_pos, dtype_mask, has_reducer;
+  PyObject *values, *indices, *outputs, *workspace, *last_used;
+  if (!PyArg_ParseTuple(args, "KKKiiiiiipO!O!O!O!O!", &launch, &workspace_bytes, &last_error, &num_args, &dispatch_pos,
+                        &ro_pos, &rows_pos, &cols_pos, &dtype_mask, &has_reducer, &PyTuple_Type, &values, &PyTuple_Type,
+                        &indices, &PyTuple_Type, &outputs, &PyDict_Type, &workspace, &PyDict_Type, &last_used))
+    return nullptr;
+  auto plan = std::make_unique<Plan>();
+  plan->launch = reinterpret_cast<LaunchFn>((uintptr_t)launch);
+  plan->workspace_bytes = reinterpret_cast<WorkspaceFn>((uintptr_t)workspace_bytes);
+  plan->last_error = reinterpret_cast<ErrorFn>((uintptr_t)last_error);
+  plan->num_args = num_args;
+  plan->dispatch_pos = dispatch_pos;
+  plan->ro_pos = ro_pos;
+  plan->rows_pos = rows_pos;
+  plan->cols_pos = cols_pos;
+  plan->dtype_mask = dtype_mask;
+  plan->has_reducer = has_reducer != 0;
+  if (PyTuple_GET_SIZE(values) > MAX_POINTERS || PyTuple_GET_SIZE(indices) > MAX_POINTERS ||
+      PyTuple_GET_SIZE(outputs) > MAX_POINTERS) {
+    PyErr_Format(PyExc_ValueError, "more than %d arguments of one kind", MAX_POINTERS);
+    return nullptr;
+  }
+  auto in_range = [&](int pos) { return pos >= 0 && pos < num_args; };
+  bool ok = in_range(dispatch_pos) && in_range(ro_pos) && in_range(rows_pos) && in_range(cols_pos);
+  for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(values); ++i) {
+    int pos, streamed, row_indexed;
+    long long dim;
+    if (!PyArg_ParseTuple(PyTuple_GET_ITEM(values, i), "iLpp", &pos, &dim, &streamed, &row_indexed)) return nullptr;
+    ok = ok && in_range(pos) && dim > 0;
+    plan->values.push_back({pos, dim, streamed != 0, row_indexed != 0});
+  }
+  for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(indices); ++i) {
+    const long pos = PyLong_AsLong(PyTuple_GET_ITEM(indices, i));
+    if (pos == -1 && PyErr_Occurred()) return nullptr;
+    ok = ok && in_range((int)pos);
+    plan->indices.push_back((int)pos);
+  }
+  for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(outputs); ++i) {
+    int lead;
+    long long dim;
+    if (!PyArg_ParseTuple(PyTuple_GET_ITEM(outputs, i), "iL", &lead, &dim)) return nullptr;
+    plan->outputs.push_back({lead, dim});
+  }
+  if (!ok) {
+    PyErr_SetString(PyExc_ValueError, "argument position out of range");
+    return nullptr;
+  }
+  Launcher* self = reinterpret_cast<Launcher*>(type->tp_alloc(type, 0));
+  if (self == nullptr) return nullptr;
+  self->plan = plan.release();
+  Py_INCREF(workspace);
+  self->workspace = workspace;
+  Py_INCREF(last_used);
+  self->last_used = last_used;
+  return reinterpret_cast<PyObject*>(self);
+}
+
+void launcher_dealloc(PyObject* self_obj) {
+  Launcher* self = reinterpret_cast<Launcher*>(self_obj);
+  delete self->plan;
+  Py_XDECREF(self->workspace);
+  Py_XDECREF(self->last_used);
+  Py_TYPE(self_obj)->tp_free(self_obj);
+}
+
+PyMethodDef launcher_methods[] = {
+    {"launch", (PyCFunction)(void (*)(void))launcher_launch, METH_FASTCALL,
+     "launch(extension, arguments): outputs, or NotImplemented when the Python path has to take the call"},
+    {nullptr, nullptr, 0, nullptr}};
+
+PyTypeObject LauncherType = {PyVarObject_HEAD_INIT(nullptr, 0)};
+
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "flexspmv_host", "Native launch path of generated FlexSpmv libraries", -1, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit_flexspmv_host() {
+  LauncherType.tp_name = "flexspmv_host.Launcher";
+  LauncherType.tp_basicsize = sizeof(Launcher);
+  LauncherType.tp_flags = Py_TPFLAGS_DEFAULT;
+  LauncherType.tp_new = launcher_new;
+  LauncherType.tp_dealloc = launcher_dealloc;
+  LauncherType.tp_methods = launcher_methods;
+  if (PyType_Ready(&LauncherType) < 0) return nullptr;
+  s_time_kernel = PyUnicode_InternFromString("time_kernel");
+  s_extra_flags = PyUnicode_InternFromString("extra_flags");
+  s_reuse_tiles = PyUnicode_InternFromString("reuse_tiles");
+  s_verify = PyUnicode_InternFromString("verify_row_aligned");
+  s_launch_count = PyUnicode_InternFromString("_launch_count");
+  if (!s_time_kernel || !s_extra_flags || !s_reuse_tiles || !s_verify || !s_launch_count) return nullptr;
+  PyObject* m = PyModule_Create(&module);
+  if (m == nullptr) return nullptr;
+  Py_INCREF(&LauncherType);
+  if (PyModule_AddObject(m, "Launcher", reinterpret_cast<PyObject*>(&LauncherType)) < 0) {
+    Py_DECREF(&LauncherType);
+    Py_DECREF(m);
+    return nullptr;
+  }
+  return m;
+}
