@@ -1035,14 +1035,14 @@ enum TileSource : int {
 // works on the current one.
 template <class G, int BLOCK, int IPT, int EPL>
 __global__ void __launch_bounds__(BLOCK)
-reduce_kernel(int2* coords, int* splits, const int source, const Tiling tl, const int num_rows,
-              const int* __restrict__ row_end, const int nnz, const typename G::Params p, int* __restrict__ carry_row,
+reduce_kernel(int2* coords, int* splits, const int* __restrict__ row_end, const int source, const int xcd_shift,
+              const int tiles, const int num_rows, const int nnz, const int nominal, const int snap_slack,
+              const int snap_mask, const int row_group, const typename G::Params p, int* __restrict__ carry_row,
               typename G::Value* __restrict__ carry_val, typename G::Value* __restrict__ agg_partials,
               unsigned* __restrict__ ticket) {
+  const Tiling tl{tiles, nominal, snap_slack, snap_mask, xcd_shift, row_group};
   const int num_tiles = tl.num_tiles;
-#ifdef FLEX_TUNE_TICKET_SUM
-  if (blockIdx.x == 0 && threadIdx.x == 0) *ticket = 0u;  // arms the last-block detection of fixup_kernel
-#endif
+  if (G::AGG_WIDTH > 0 && blockIdx.x == 0 && threadIdx.x == 0) *ticket = 0u;  // for the fixup_kernel of this launch
 #ifdef FLEX_TUNE_PERSISTENT
   int tile = blockIdx.x;
   if (tile >= num_tiles) return;
@@ -1203,28 +1203,104 @@ flat_kernel(const typename G::Params p, const int nnz, const int num_tiles,
 
 // ----------------------------------------------------------------------------------------------
 // Fix-up: fold tile carries into their rows (tile order) and reduce the aggregator partials.
-// Tiles are handled in chunks of BLOCK, a thread per tile.  A run of tiles that carry into the same row is
-// summed by a block-wide segmented scan (wave64 DPP scan, then a fold across the wavefronts in order); the
-// thread of the run's last tile adds the total to the row.  A run that starts in the chunk and goes on
-// beyond it - a row of millions of non-zeros - is finished by the whole block: it walks the following
-// tiles BLOCK at a time for as long as they carry into that row and adds them up in a fixed order; the
-// chunks those tiles belong to see that their leading tiles continue an earlier run and leave them alone.
-// Nothing here depends on timing: the same sums in the same order on every run, no atomics.
-// The aggregator partials (PARTS_PER_TILE per tile: one, or one per wavefront of the reducer block) are summed in a
-// fixed order.
-//   SINGLE = false: block b handles tiles [b*BLOCK, (b+1)*BLOCK) and leaves its aggregator sum in
-//                   block_partials[b]; aggregate_kernel adds those, again in a fixed order.
-//   SINGLE = true:  one block walks all chunks (launches of a few thousand tiles) and assigns the
-//                   aggregator outputs itself: one kernel less.
-// (Finishing the sum in the last fix-up block to finish, found with a ticket counter - FLEX_TUNE_TICKET_SUM -,
-// was measured twice and is slower, also with the row outputs stored non-temporally: Poisson 256^3 step
-// 323.0 us against 319.0; each block's release at device scope costs more than the 4.6 us kernel it saves.)
+//
+// Nothing here is about bytes: the kernel is a chain of memory latencies behind the reducer (an empty kernel costs
+// 1.5 us there), so it is written for few links.  A block takes BLOCK * per tiles, `per` a thread, and loads all their
+// carry rows and partials at once; a vote says what there is to do:
+//   no carry (row-snapped launches)       nothing;
+//   no run of more than one tile          each carry and its row's current value are loaded together, added, stored;
+//   a run of tiles that carry into one row  the block walks its tiles in chunks of BLOCK and sums the run by a segmented
+//       scan (wave64 DPP scan, then a fold across the wavefronts in order); the thread of the run's last tile adds the
+//       total to the row.  A run that starts in the chunk and goes on beyond it - a row of millions of non-zeros - is
+//       finished by the whole block: it walks the following tiles BLOCK at a time for as long as they carry into that
+//       row and adds them up in a fixed order; the chunks those tiles belong to see that their leading tiles continue an
+//       earlier run and leave them alone.
+// The same sums in the same order on every run, no floating-point atomics.
+//
+// Launches of a few thousand tiles use one block of 1024 threads.  Larger ones use blocks of 256 threads: a tile per
+// thread where tiles carry (runs are common there, and blocks walk them side by side), eight per thread on row-snapped
+// launches.  With several blocks the one that draws the last ticket adds the blocks' aggregator sums, in block order.
+// What it reads was stored write-through at device scope and had arrived before the ticket was drawn, so no block
+// has to write its XCD's L2 back: that release cost 15 us a launch, a kernel of its own for the sum 4.7.
+// Whole passes, against loads one tile after the other and the sum in a kernel of its own: spring-mass 100^3 25.9 ->
+// 25.0 us, rows of 18 to 81 entries (301 000 of them, float64) 43.5 -> 42.7, Poisson 256^3 308.6 -> 308.3.
 // ----------------------------------------------------------------------------------------------
-template <class G, int BLOCK, int PARTS_PER_TILE, bool SINGLE>
+
+// One pass over the block's tiles; returns whether the block has runs to walk.  acc: the thread's share of the
+// aggregators.
+template <class G, int BLOCK, int PARTS_PER_TILE, int PER>
+__device__ __forceinline__ bool
+fold_single_carries(const typename G::Params& p, const int first, const int num_tiles, const int* __restrict__ carry_row,
+                    const typename G::Value* __restrict__ carry_val, const typename G::Value* __restrict__ agg_partials,
+                    int* s_vote, Pack<typename G::Value, G::AGG_WIDTH>& acc) {
+  using V = typename G::Value;
+  constexpr int RED = G::RED_WIDTH, AGG = G::AGG_WIDTH;
+  constexpr int NW = BLOCK / WAVE;
+  constexpr int PARTS = AGG > 0 ? PARTS_PER_TILE * AGG : 1;
+  const int tid = threadIdx.x;
+  const int last = num_tiles - 1;
+  int row[PER], before[PER], after[PER];
+  V part[PER][PARTS];
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    const int t = min(first + i * BLOCK + tid, last);
+    row[i] = carry_row[t];
+    before[i] = carry_row[max(t - 1, 0)];
+    after[i] = carry_row[min(t + 1, last)];
+#pragma unroll
+    for (int c = 0; c < (AGG > 0 ? PARTS : 0); ++c) part[i][c] = agg_partials[(size_t)t * PARTS + c];
+  }
+  bool any = false, runs = false;
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    const int t = first + i * BLOCK + tid;
+    if (t > last) row[i] = -1;
+    any |= row[i] >= 0;
+    runs |= row[i] >= 0 && t < last && after[i] == row[i];
+    if (t > 0 && before[i] == row[i]) row[i] = -1;  // belongs to a run whose first tile another thread (or block) has
+#pragma unroll
+    for (int c = 0; c < (AGG > 0 ? PARTS : 0); ++c) acc.v[c % (AGG > 0 ? AGG : 1)] += t <= last ? part[i][c] : V(0);
+  }
+  if constexpr (RED > 0) {
+    const int mine = (__builtin_amdgcn_ballot_w64(any) != 0ull ? 1 : 0) | (__builtin_amdgcn_ballot_w64(runs) != 0ull ? 2 : 0);
+    if ((tid & (WAVE - 1)) == 0) s_vote[tid / WAVE] = mine;
+    __syncthreads();
+    int vote = 0;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) vote |= s_vote[w];
+    if (vote == 0) return false;
+    if ((vote & 2) != 0) return true;
+    constexpr int WORDS = RED * (int)(sizeof(V) / 4);
+    constexpr int TOGETHER = WORDS * PER <= 16 ? PER : (WORDS >= 16 ? 1 : 16 / WORDS);  // within 32 registers
+    for (int i0 = 0; i0 < PER; i0 += TOGETHER) {
+      Pack<V, RED> sum[TOGETHER], now[TOGETHER];
+#pragma unroll
+      for (int k = 0; k < TOGETHER; ++k) {
+        const int i = min(i0 + k, PER - 1);
+        const int t = min(first + i * BLOCK + tid, last);
+#pragma unroll
+        for (int c = 0; c < RED; ++c) sum[k].v[c] = carry_val[(size_t)t * RED + c];
+        G::current_row(p, max(row[i], 0), now[k]);
+      }
+#pragma unroll
+      for (int k = 0; k < TOGETHER; ++k) {
+        const int i = i0 + k;
+        if (i < PER && row[i < PER ? i : 0] >= 0) {
+#pragma unroll
+          for (int c = 0; c < RED; ++c) now[k].v[c] += sum[k].v[c];
+          G::store_row(p, row[i < PER ? i : 0], now[k]);
+        }
+      }
+    }
+  }
+  return false;
+}
+
+template <class G, int BLOCK, int PARTS_PER_TILE>
 __global__ void __launch_bounds__(BLOCK)
-fixup_kernel(const typename G::Params p, const int num_tiles, const int* __restrict__ carry_row,
-             const typename G::Value* __restrict__ carry_val, const typename G::Value* __restrict__ agg_partials,
-             typename G::Value* __restrict__ block_partials, unsigned* __restrict__ ticket) {
+fixup_kernel(const int* __restrict__ carry_row, const typename G::Value* __restrict__ agg_partials,
+             const typename G::Value* __restrict__ carry_val, const int num_tiles, const int per,
+             typename G::Value* __restrict__ block_partials, unsigned* __restrict__ ticket, const typename G::Params p) {
   using V = typename G::Value;
   constexpr int RED = G::RED_WIDTH, AGG = G::AGG_WIDTH;
   constexpr int REDN = RED > 0 ? RED : 1;
@@ -1232,256 +1308,179 @@ fixup_kernel(const typename G::Params p, const int num_tiles, const int* __restr
   const int tid = threadIdx.x;
   const int lane = tid & (WAVE - 1);
   const int wave = tid / WAVE;
+  __shared__ int s_vote[NW];
   __shared__ int s_key[NW];
   __shared__ V s_val[NW][REDN];
   __shared__ int s_trail_row;
   __shared__ V s_trail_val[REDN];
   Pack<V, AGG> acc;
   zero(acc);
-  const int first_chunk = SINGLE ? 0 : (int)blockIdx.x * BLOCK;
-  const int chunk_step = SINGLE ? BLOCK : num_tiles;  // not SINGLE: one chunk per block
-  // One block for all chunks: one pass with all loads in flight together sums the aggregator partials and
-  // looks whether any run is longer than a tile.  If none is (always on row-snapped launches, where no
-  // tile carries at all), every carry goes to its row as it is and the chunk loop below is skipped.
-  bool may_have_runs = true;
-  bool partials_done = false;
-  if constexpr (SINGLE) {
-    constexpr int KEPT = 4;  // carries a thread keeps in registers between the two phases
-    int kept_row[KEPT];
-    bool multi = false;
-    for (int i = 0, t = tid; t < num_tiles; ++i, t += BLOCK) {
-      if constexpr (RED > 0) {
-        const int row = carry_row[t];
-        const int next_row = (t + 1 < num_tiles) ? carry_row[t + 1] : -2;
-        multi |= (row >= 0 && next_row == row);
-        if (i < KEPT) kept_row[i] = row;
-      }
-      if constexpr (AGG > 0) {
-#pragma unroll
-        for (int w = 0; w < PARTS_PER_TILE; ++w) {
-#pragma unroll
-          for (int c = 0; c < AGG; ++c) acc.v[c] += agg_partials[((size_t)t * PARTS_PER_TILE + w) * AGG + c];
-        }
-      }
-    }
-    partials_done = true;
-    if constexpr (RED > 0) {
-      may_have_runs = __syncthreads_or(multi ? 1 : 0) != 0;
-      if (!may_have_runs) {
-        for (int i = 0, t = tid; t < num_tiles; ++i, t += BLOCK) {
-          const int row = (i < KEPT) ? kept_row[i] : carry_row[t];
-          if (row >= 0 && !(t > 0 && carry_row[t - 1] == row)) {
-            Pack<V, RED> sum;
-#pragma unroll
-            for (int c = 0; c < RED; ++c) sum.v[c] = carry_val[(size_t)t * RED + c];
-            G::add_row(p, row, sum);
-          }
-        }
-      }
-    } else {
-      may_have_runs = false;
-    }
-  }
-  for (int chunk = first_chunk; chunk < num_tiles && (!SINGLE || may_have_runs); chunk += chunk_step) {
-    const int t = chunk + tid;
-    const bool valid = t < num_tiles;
-    if constexpr (RED > 0) {
+  const int first = (int)blockIdx.x * BLOCK * per;
+  auto fold = [&](auto per_tag) {
+    return fold_single_carries<G, BLOCK, PARTS_PER_TILE, decltype(per_tag)::value>(p, first, num_tiles, carry_row, carry_val,
+                                                                                   agg_partials, s_vote, acc);
+  };
+  const bool runs = per == 1 ? fold(std::integral_constant<int, 1>{})   // uniform over the launch
+                    : per == 2 ? fold(std::integral_constant<int, 2>{})
+                    : per <= 4 ? fold(std::integral_constant<int, 4>{})
+                               : fold(std::integral_constant<int, 8>{});
+  if constexpr (RED > 0) {
+    for (int chunk = first; runs && chunk < min(first + BLOCK * per, num_tiles); chunk += BLOCK) {
+      const int t = chunk + tid;
+      const bool valid = t < num_tiles;
       const int row = valid ? carry_row[t] : -1;
       const int next_row = (valid && t + 1 < num_tiles) ? carry_row[t + 1] : -2;
       V run[REDN];
 #pragma unroll
       for (int c = 0; c < RED; ++c) run[c] = (row >= 0) ? carry_val[(size_t)t * RED + c] : V(0);
-      // Most chunks have no run of more than one tile (none at all on row-snapped launches): then a tile's
-      // carry goes to its row as it is, unless the tile continues a run that an earlier chunk owns.
-      if (!may_have_runs || !__syncthreads_or((row >= 0 && next_row == row) ? 1 : 0)) {
-        if (row >= 0 && !(t > 0 && carry_row[t - 1] == row)) {
+      // does the chunk start inside a run that an earlier chunk owns?
+      const int chunk_first_row = carry_row[chunk];
+      const bool leading_continues = chunk > 0 && chunk_first_row >= 0 && carry_row[chunk - 1] == chunk_first_row;
+      // segmented inclusive sums over the chunk, keyed by row (equal rows are contiguous)
+      wave_segmented_inclusive_sum<V, REDN>(row, run);
+      if (tid == 0) s_trail_row = -1;
+      if (lane == WAVE - 1) {
+        s_key[wave] = row;
+#pragma unroll
+        for (int c = 0; c < RED; ++c) s_val[wave][c] = run[c];
+      }
+      __syncthreads();
+      {
+        int pk = -3;
+        V pv[REDN];
+#pragma unroll
+        for (int c = 0; c < RED; ++c) pv[c] = V(0);
+#pragma unroll
+        for (int w = 0; w < NW - 1; ++w) {
+          if (w < wave) {
+            const int k = s_key[w];
+#pragma unroll
+            for (int c = 0; c < RED; ++c) pv[c] = (k == pk) ? static_cast<V>(pv[c] + s_val[w][c]) : s_val[w][c];
+            pk = k;
+          }
+        }
+        if (wave > 0 && row >= 0 && row == pk) {  // my run began in an earlier wavefront of this chunk
+#pragma unroll
+          for (int c = 0; c < RED; ++c) run[c] += pv[c];
+        }
+      }
+      const bool mine = row >= 0 && !(leading_continues && row == chunk_first_row);
+      const bool part_end = next_row != row || tid == BLOCK - 1;  // last tile of the run inside this chunk
+      if (mine && part_end) {
+        if (next_row != row) {  // the run ends here
           Pack<V, RED> sum;
 #pragma unroll
           for (int c = 0; c < RED; ++c) sum.v[c] = run[c];
           G::add_row(p, row, sum);
+        } else {  // it goes on in the following chunks: the block finishes it together
+          s_trail_row = row;
+#pragma unroll
+          for (int c = 0; c < RED; ++c) s_trail_val[c] = run[c];
         }
-      } else {
-        // does the chunk start inside a run that an earlier chunk owns?
-        const int chunk_first_row = carry_row[chunk];
-        const bool leading_continues = chunk > 0 && chunk_first_row >= 0 && carry_row[chunk - 1] == chunk_first_row;
-        // segmented inclusive sums over the chunk, keyed by row (equal rows are contiguous)
-        wave_segmented_inclusive_sum<V, REDN>(row, run);
-        if (tid == 0) s_trail_row = -1;
+      }
+      __syncthreads();
+      const int trail_row = s_trail_row;
+      if (trail_row >= 0) {  // uniform
+        V ext[REDN];
+#pragma unroll
+        for (int c = 0; c < RED; ++c) ext[c] = V(0);
+        // EXT_STEP chunks per vote, all their loads in flight together (the values are fetched whether or
+        // not the tile belongs to the run: a load under the test would wait for the row first)
+        constexpr int EXT_STEP = 4;
+        const int last_tile = num_tiles - 1;
+        for (int base = chunk + BLOCK; base < num_tiles; base += EXT_STEP * BLOCK) {
+          int urow[EXT_STEP];
+          V uval[EXT_STEP][REDN];
+#pragma unroll
+          for (int k = 0; k < EXT_STEP; ++k) {
+            const int u = min(base + k * BLOCK + tid, last_tile);
+            urow[k] = carry_row[u];
+#pragma unroll
+            for (int c = 0; c < RED; ++c) uval[k][c] = carry_val[(size_t)u * RED + c];
+          }
+          bool all_same = true;
+#pragma unroll
+          for (int k = 0; k < EXT_STEP; ++k) {
+            const bool same = base + k * BLOCK + tid < num_tiles && urow[k] == trail_row;
+            all_same &= same;
+            if (same) {
+#pragma unroll
+              for (int c = 0; c < RED; ++c) ext[c] += uval[k][c];
+            }
+          }
+          if (!__syncthreads_and(all_same ? 1 : 0)) break;  // the run is contiguous: a mismatch ends it
+        }
+        wave_sum_to_last_lane<V, REDN>(ext);
+        __syncthreads();  // s_val is free again
         if (lane == WAVE - 1) {
-          s_key[wave] = row;
 #pragma unroll
-          for (int c = 0; c < RED; ++c) s_val[wave][c] = run[c];
+          for (int c = 0; c < RED; ++c) s_val[wave][c] = ext[c];
         }
         __syncthreads();
-        {
-          int pk = -3;
-          V pv[REDN];
+        if (tid == 0) {
+          Pack<V, RED> sum;
 #pragma unroll
-          for (int c = 0; c < RED; ++c) pv[c] = V(0);
-          for (int w = 0; w < NW - 1; ++w) {
-            if (w < wave) {
-              const int k = s_key[w];
+          for (int c = 0; c < RED; ++c) {
+            V x = s_trail_val[c];
 #pragma unroll
-              for (int c = 0; c < RED; ++c) pv[c] = (k == pk) ? static_cast<V>(pv[c] + s_val[w][c]) : s_val[w][c];
-              pk = k;
-            }
+            for (int w = 0; w < NW; ++w) x += s_val[w][c];
+            sum.v[c] = x;
           }
-          if (wave > 0 && row >= 0 && row == pk) {  // my run began in an earlier wavefront of this chunk
-#pragma unroll
-            for (int c = 0; c < RED; ++c) run[c] += pv[c];
-          }
-        }
-        const bool mine = row >= 0 && !(leading_continues && row == chunk_first_row);
-        const bool part_end = next_row != row || tid == BLOCK - 1;  // last tile of the run inside this chunk
-        if (mine && part_end) {
-          if (next_row != row) {  // the run ends here
-            Pack<V, RED> sum;
-#pragma unroll
-            for (int c = 0; c < RED; ++c) sum.v[c] = run[c];
-            G::add_row(p, row, sum);
-          } else {  // it goes on in the following chunks: the block finishes it together
-            s_trail_row = row;
-#pragma unroll
-            for (int c = 0; c < RED; ++c) s_trail_val[c] = run[c];
-          }
-        }
-        __syncthreads();
-        const int trail_row = s_trail_row;
-        if (trail_row >= 0) {  // uniform
-          V ext[REDN];
-#pragma unroll
-          for (int c = 0; c < RED; ++c) ext[c] = V(0);
-          // EXT_STEP chunks per vote, all their loads in flight together (the values are fetched whether or
-          // not the tile belongs to the run: a load under the test would wait for the row first)
-          constexpr int EXT_STEP = 4;
-          const int last_tile = num_tiles - 1;
-          for (int base = chunk + BLOCK; base < num_tiles; base += EXT_STEP * BLOCK) {
-            int urow[EXT_STEP];
-            V uval[EXT_STEP][REDN];
-#pragma unroll
-            for (int k = 0; k < EXT_STEP; ++k) {
-              const int u = min(base + k * BLOCK + tid, last_tile);
-              urow[k] = carry_row[u];
-#pragma unroll
-              for (int c = 0; c < RED; ++c) uval[k][c] = carry_val[(size_t)u * RED + c];
-            }
-            bool all_same = true;
-#pragma unroll
-            for (int k = 0; k < EXT_STEP; ++k) {
-              const bool same = base + k * BLOCK + tid < num_tiles && urow[k] == trail_row;
-              all_same &= same;
-              if (same) {
-#pragma unroll
-                for (int c = 0; c < RED; ++c) ext[c] += uval[k][c];
-              }
-            }
-            if (!__syncthreads_and(all_same ? 1 : 0)) break;  // the run is contiguous: a mismatch ends it
-          }
-          wave_sum_to_last_lane<V, REDN>(ext);
-          __syncthreads();  // s_val is free again
-          if (lane == WAVE - 1) {
-#pragma unroll
-            for (int c = 0; c < RED; ++c) s_val[wave][c] = ext[c];
-          }
-          __syncthreads();
-          if (tid == 0) {
-            Pack<V, RED> sum;
-#pragma unroll
-            for (int c = 0; c < RED; ++c) {
-              V x = s_trail_val[c];
-              for (int w = 0; w < NW; ++w) x += s_val[w][c];
-              sum.v[c] = x;
-            }
-            G::add_row(p, trail_row, sum);
-          }
-        }
-        __syncthreads();  // before the next chunk reuses the shared arrays
-      }
-    }
-    if constexpr (AGG > 0) {
-      if (valid && !partials_done) {
-#pragma unroll
-        for (int w = 0; w < PARTS_PER_TILE; ++w) {
-#pragma unroll
-          for (int c = 0; c < AGG; ++c) acc.v[c] += agg_partials[((size_t)t * PARTS_PER_TILE + w) * AGG + c];
+          G::add_row(p, trail_row, sum);
         }
       }
+      __syncthreads();  // before the next chunk reuses the shared arrays
     }
   }
   if constexpr (AGG > 0) {
     __shared__ V s_wave_agg[NW][AGG];
     __shared__ int s_is_last;
-    (void)s_is_last;
-    wave_sum_to_last_lane<V, AGG>(acc.v);
-    if (lane == WAVE - 1) {
+    auto block_total = [&](Pack<V, AGG>& share) {  // the block's sum, in thread 0
+      wave_sum_to_last_lane<V, AGG>(share.v);
+      if (lane == WAVE - 1) {
 #pragma unroll
-      for (int c = 0; c < AGG; ++c) s_wave_agg[wave][c] = acc.v[c];
-    }
-    __syncthreads();
-    if (tid == 0) {
+        for (int c = 0; c < AGG; ++c) s_wave_agg[wave][c] = share.v[c];
+      }
+      __syncthreads();
       Pack<V, AGG> total;
 #pragma unroll
       for (int c = 0; c < AGG; ++c) {
         V s = s_wave_agg[0][c];
+#pragma unroll
         for (int w = 1; w < NW; ++w) s += s_wave_agg[w][c];
         total.v[c] = s;
       }
-      if constexpr (SINGLE) {
-        G::store_agg(p, total);
-      } else {
-#ifdef FLEX_TUNE_TICKET_SUM
-        // tuning switch (measured slower, see fixup_kernel's header): the block that draws the last ticket adds the
-        // blocks' partials itself.  Each block publishes its partial before it takes a ticket (release at device
-        // scope), the last one acquires after taking its own.  The reducer kernel zeroes the ticket.
+      return total;
+    };
+    const Pack<V, AGG> total = block_total(acc);
+    if (gridDim.x == 1) {
+      if (tid == 0) G::store_agg(p, total);
+      return;
+    }
+    if (tid == 0) {
+#pragma unroll
+      for (int c = 0; c < AGG; ++c)
+        __hip_atomic_store(&block_partials[(size_t)blockIdx.x * AGG + c], total.v[c], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the stores above have arrived before the ticket is drawn
+      s_is_last = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1 ? 1 : 0;
+    }
+    __syncthreads();
+    if (s_is_last) {
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+      Pack<V, AGG> share;
+      zero(share);
+      for (int j = tid; j < (int)gridDim.x; j += BLOCK) {
 #pragma unroll
         for (int c = 0; c < AGG; ++c)
-          __hip_atomic_store(&block_partials[(size_t)blockIdx.x * AGG + c], total.v[c], __ATOMIC_RELAXED,
-                             __HIP_MEMORY_SCOPE_AGENT);
-        __atomic_thread_fence(__ATOMIC_RELEASE);
-        const unsigned drawn = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
-        s_is_last = (drawn == gridDim.x - 1) ? 1 : 0;
-#else
-#pragma unroll
-        for (int c = 0; c < AGG; ++c) block_partials[(size_t)blockIdx.x * AGG + c] = total.v[c];
-#endif
+          share.v[c] += __hip_atomic_load(&block_partials[(size_t)j * AGG + c], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       }
+      const Pack<V, AGG> all = block_total(share);
+      if (tid == 0) G::store_agg(p, all);
     }
-#ifdef FLEX_TUNE_TICKET_SUM
-    if constexpr (!SINGLE) {
-      __syncthreads();
-      if (s_is_last) {
-        __atomic_thread_fence(__ATOMIC_ACQUIRE);
-        Pack<V, AGG> fin;
-        zero(fin);
-        for (int j = tid; j < (int)gridDim.x; j += BLOCK) {
-#pragma unroll
-          for (int c = 0; c < AGG; ++c)
-            fin.v[c] += __hip_atomic_load(&block_partials[(size_t)j * AGG + c], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-        wave_sum_to_last_lane<V, AGG>(fin.v);
-        __syncthreads();
-        if (lane == WAVE - 1) {
-#pragma unroll
-          for (int c = 0; c < AGG; ++c) s_wave_agg[wave][c] = fin.v[c];
-        }
-        __syncthreads();
-        if (tid == 0) {
-          Pack<V, AGG> total;
-#pragma unroll
-          for (int c = 0; c < AGG; ++c) {
-            V t = s_wave_agg[0][c];
-            for (int w = 1; w < NW; ++w) t += s_wave_agg[w][c];
-            total.v[c] = t;
-          }
-          G::store_agg(p, total);
-        }
-      }
-    }
-#endif
   }
 }
 
-// Final aggregator sum: one block adds `count` partial vectors in a fixed order and assigns the
+// Final aggregator sum of a flat launch: one block adds `count` partial vectors in a fixed order and assigns the
 // outputs (the reference assigns too: cpu_template/merged_spmv_template_aggregator.h:75-87).
 template <class G, int BLOCK>
 __global__ void __launch_bounds__(BLOCK)

@@ -168,9 +168,9 @@ struct Dispatch {
     Tiling tiling;
     int num_tiles;
     int flat_blocks;
-    int carry_blocks;
     bool search_in_blocks;
     bool single_fixup;
+    int fixup_per, fixup_blocks;  // tiles per thread of fixup_kernel, its blocks
     size_t off_coords, off_splits, off_carry_row, off_carry_val, off_partials, off_block_partials, off_ticket, total;
   };
 
@@ -237,7 +237,8 @@ struct Dispatch {
     l.search_in_blocks = REDUCER && l.num_tiles <= FLEX_TUNE_INBLOCK_MAX_TILES;
     // ... twice as many where tiles start on rows: hardly a tile carries then, and the block only walks the records
     // (spring-mass 100^3, 4 606 tiles: 2.6 us; with a carry per tile 8 192 tiles cost one block 20 us)
-    l.single_fixup = REDUCER && l.num_tiles <= FLEX_TUNE_SINGLE_FIXUP_MAX_TILES * (l.tiling.snap_slack > 0 ? 2 : 1);
+    l.single_fixup = REDUCER && l.num_tiles <= FLEX_TUNE_SINGLE_FIXUP_MAX_TILES * (l.tiling.snap_slack > 0 ? 2 : 1) &&
+                     l.num_tiles <= 8 * SINGLE_FIXUP_BLOCK;
     size_t off = 0;
     l.off_coords = off;
     if (REDUCER) off += align_up(sizeof(int2) * ((size_t)l.num_tiles + 1));
@@ -247,16 +248,18 @@ struct Dispatch {
     if (REDUCER) off += align_up(sizeof(int) * (size_t)l.num_tiles);
     l.off_carry_val = off;
     if (REDUCER) off += align_up(sizeof(V) * (size_t)l.num_tiles * (G::RED_WIDTH > 0 ? G::RED_WIDTH : 1));
-    l.carry_blocks = (l.num_tiles + FIXUP_BLOCK - 1) / FIXUP_BLOCK;
+    // (fixup_kernel: one block takes up to 8 tiles per thread; several blocks one, or eight where tiles hardly carry)
+    if (l.single_fixup) l.fixup_per = (l.num_tiles + SINGLE_FIXUP_BLOCK - 1) / SINGLE_FIXUP_BLOCK;
+    else l.fixup_per = l.tiling.snap_slack > 0 ? 8 : 1;
+    const int per_block = (l.single_fixup ? SINGLE_FIXUP_BLOCK : FIXUP_BLOCK) * l.fixup_per;
+    l.fixup_blocks = (l.num_tiles + per_block - 1) / per_block;
     l.off_partials = off;
     const size_t parts = REDUCER ? (size_t)l.num_tiles * partials_per_tile<BLOCK>() : (size_t)MAX_PERSISTENT_BLOCKS;
     if (G::AGG_WIDTH > 0) off += align_up(sizeof(V) * parts * G::AGG_WIDTH);
     l.off_block_partials = off;
-    if (REDUCER && G::AGG_WIDTH > 0) off += align_up(sizeof(V) * (size_t)l.carry_blocks * G::AGG_WIDTH);
+    if (REDUCER && G::AGG_WIDTH > 0) off += align_up(sizeof(V) * (size_t)l.fixup_blocks * G::AGG_WIDTH);
     l.off_ticket = off;
-#ifdef FLEX_TUNE_TICKET_SUM
-    off += align_up(sizeof(unsigned));
-#endif
+    if (REDUCER && G::AGG_WIDTH > 0) off += align_up(sizeof(unsigned));
     l.total = off;
     return true;
   }
@@ -380,14 +383,17 @@ struct Dispatch {
       // launches with short regular rows (row-snapped tiles) take several neighbouring edges per load
       constexpr int EPL = edges_per_load<G, IPT>();
       const bool wide_loads = EPL > 1 && l.tiling.snap_slack > 0 && nnz >= EPL;
+      const Tiling& tl = l.tiling;
       auto launch_reducer = [&](auto kernel, const char* name) {
         if (timed) {
           hipExtLaunchKernelGGL(kernel, dim3(reduce_grid), dim3(BLOCK), 0, stream, g_timer.start, g_timer.stop, 0, coords,
-                                splits, source, l.tiling, num_rows, row_end, nnz, p, carry_row, carry_val, partials, ticket);
+                                splits, row_end, source, tl.xcd_shift, tl.num_tiles, num_rows, nnz, tl.nominal,
+                                tl.snap_slack, tl.snap_mask, tl.row_group, p, carry_row, carry_val, partials, ticket);
           g_timer.armed = true;
         } else {
-          hipLaunchKernelGGL(kernel, dim3(reduce_grid), dim3(BLOCK), 0, stream, coords, splits, source, l.tiling, num_rows,
-                             row_end, nnz, p, carry_row, carry_val, partials, ticket);
+          hipLaunchKernelGGL(kernel, dim3(reduce_grid), dim3(BLOCK), 0, stream, coords, splits, row_end, source,
+                             tl.xcd_shift, tl.num_tiles, num_rows, nnz, tl.nominal, tl.snap_slack, tl.snap_mask,
+                             tl.row_group, p, carry_row, carry_val, partials, ticket);
         }
         report(name, kernel, reduce_grid, BLOCK);
       };
@@ -395,24 +401,13 @@ struct Dispatch {
       else launch_reducer(reduce_kernel<G, BLOCK, IPT, 1>, "reduce_kernel");
       V* block_partials = (V*)(ws + l.off_block_partials);
       constexpr int PARTS = partials_per_tile<BLOCK>();
-      if (l.single_fixup) {
-        hipLaunchKernelGGL((fixup_kernel<G, SINGLE_FIXUP_BLOCK, PARTS, true>), dim3(1), dim3(SINGLE_FIXUP_BLOCK), 0,
-                           stream, p, l.num_tiles, (const int*)carry_row, (const V*)carry_val, (const V*)partials,
-                           block_partials, ticket);
-        report("fixup_kernel (one block)", fixup_kernel<G, SINGLE_FIXUP_BLOCK, PARTS, true>, 1, SINGLE_FIXUP_BLOCK);
-      } else {
-        hipLaunchKernelGGL((fixup_kernel<G, FIXUP_BLOCK, PARTS, false>), dim3(l.carry_blocks), dim3(FIXUP_BLOCK), 0,
-                           stream, p, l.num_tiles, (const int*)carry_row, (const V*)carry_val, (const V*)partials,
-                           block_partials, ticket);
-        report("fixup_kernel", fixup_kernel<G, FIXUP_BLOCK, PARTS, false>, l.carry_blocks, FIXUP_BLOCK);
-#ifndef FLEX_TUNE_TICKET_SUM
-        if (G::AGG_WIDTH > 0) {
-          hipLaunchKernelGGL((aggregate_kernel<G, FIXUP_BLOCK>), dim3(1), dim3(FIXUP_BLOCK), 0, stream, p,
-                             (const V*)block_partials, l.carry_blocks);
-          report("aggregate_kernel", aggregate_kernel<G, FIXUP_BLOCK>, 1, FIXUP_BLOCK);
-        }
-#endif
-      }
+      auto launch_fixup = [&](auto kernel, const int block, const char* name) {
+        hipLaunchKernelGGL(kernel, dim3(l.fixup_blocks), dim3(block), 0, stream, (const int*)carry_row,
+                           (const V*)partials, (const V*)carry_val, l.num_tiles, l.fixup_per, block_partials, ticket, p);
+        report(name, kernel, l.fixup_blocks, block);
+      };
+      if (l.single_fixup) launch_fixup(fixup_kernel<G, SINGLE_FIXUP_BLOCK, PARTS>, SINGLE_FIXUP_BLOCK, "fixup_kernel (one block)");
+      else launch_fixup(fixup_kernel<G, FIXUP_BLOCK, PARTS>, FIXUP_BLOCK, "fixup_kernel");
     } else {
       int grid = resident_grid(flat_kernel<G, BLOCK, IPT>, BLOCK, grid_cache);
       if (grid > l.num_tiles) grid = l.num_tiles;
