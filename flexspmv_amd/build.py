@@ -33,6 +33,9 @@ HIPCC_FLAGS = [
     f"--offload-arch={OFFLOAD_ARCH}", "-O3", "-std=c++17", "-fPIC", "-shared",
     # packed-FP32 instructions are kept out of every kernel of this package
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+    # the first 14 words of a kernel's arguments arrive in scalar registers instead of being loaded by its first
+    # instructions: 0.6 - 1 us less of every launch (61 x 47 x 83 stencil 9.3 -> 8.6 us, spring-mass 100^3 25.0 -> 24.1)
+    "-mllvm", "-amdgpu-kernarg-preload-count=14",
     "-Wno-unused-command-line-argument", "-Wno-unknown-warning-option",
 ]
 
