@@ -61,6 +61,7 @@ class LaunchArgs(ctypes.Structure):
         ("workspace_bytes", ctypes.c_size_t),
         ("stream", ctypes.c_void_p),
         ("flags", ctypes.c_uint32),
+        ("counters", ctypes.c_void_p),
     ]
 
 
@@ -347,11 +348,13 @@ class HipExtension:
         return rep
 
     def merged_spmv_launch(self, *args, **kwargs):
-        # A library's first launch, and what the native path does not take (it says so before it has done anything:
-        # keywords, a failed check, a stream capture, timing and debugging options), go through Python.
-        if self._launch_count and not kwargs:
+        # What the native path does not take (it says so before it has done anything: keywords, a failed check, a
+        # stream capture, timing and debugging options) goes through Python.
+        if not kwargs:
             outs = self._native(self, args)
             if outs is not NotImplemented:
+                if self._launch_count == 1:       # the record of a library's first launch (_same_arguments)
+                    self._remember_call(args, outs)
                 return outs
         return self._launch_checked(args, kwargs)
 
@@ -472,6 +475,16 @@ class HipExtension:
         rep.ws_bytes = ws_bytes
         rep.out_shapes = tuple(tuple(o.shape) for o in outs)
         self._call_state().repeat = rep
+
+    def _remember_call(self, args, outs):
+        import torch
+        where = {n: i for i, n in enumerate(self._param_names)}
+        dispatch = args[where[self._dispatch_name]]
+        num_rows, num_cols = args[where["num_rows"]], args[where["num_cols"]]
+        ne = args[where[self._index_names[0]]].numel() if self._index_names else num_cols
+        dt = _TORCH_DTYPE_NAMES()[dispatch.dtype]
+        self._remember(args, outs or (), num_rows, num_cols, ne, dt, dispatch.dtype, dispatch.device,
+                       self.workspace_bytes(dt, num_rows, ne))
 
     def _launch(self, values, indices, outs, ro, num_rows, num_cols, ne, dt, device, index, ws_bytes):
         """Fill the argument block and call the library on the current stream of the (current) device."""

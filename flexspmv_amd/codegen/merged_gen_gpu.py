@@ -334,10 +334,11 @@ def generate_hip_source(ir: FusedGraphIR, dtypes: Optional[Sequence[str]] = None
         body += [f"q_agg.v[{first + c}] = {_component(v, c % v.dim)};" for c in range(dim)]
     edge_pure = not any("stream_store(" in line for line in body)
 
-    store_row, add_row, current_row, store_agg = [], [], [], []
+    store_row, store_row_through, add_row, current_row, store_agg = [], [], [], [], []
     for (rname, first, dim) in kp.red_slices:
         for c in range(dim):
             store_row.append(f"flex::stream_store(q_p.output_y_{rname}_ptr + (size_t)q_row * {dim} + {c}, q_tot.v[{first + c}]);")
+            store_row_through.append(f"flex::through_store(q_p.output_y_{rname}_ptr + (size_t)q_row * {dim} + {c}, q_tot.v[{first + c}]);")
             current_row.append(f"q_now.v[{first + c}] = q_p.output_y_{rname}_ptr[(size_t)q_row * {dim} + {c}];")
             add_row.append(f"q_p.output_y_{rname}_ptr[(size_t)q_row * {dim} + {c}] += q_tot.v[{first + c}];")
     for (gname, first, dim) in kp.agg_slices:
@@ -445,6 +446,9 @@ struct Graph {{
   template <class T>
   static FLEX_DEV void store_row(const Params& q_p, const int q_row, const T& q_tot) {{
 {_indent(store_row)}  }}
+  template <class T>
+  static FLEX_DEV void store_row_through(const Params& q_p, const int q_row, const T& q_tot) {{
+{_indent(store_row_through)}  }}
   template <class T>
   static FLEX_DEV void add_row(const Params& q_p, const int q_row, const T& q_tot) {{
 {_indent(add_row)}  }}

@@ -78,6 +78,23 @@ template <typename T> __device__ __forceinline__ void stream_store(T* p, T v) { 
 template <typename T> __device__ __forceinline__ void stream_store(T* p, T v) { __builtin_nontemporal_store(v, p); }
 #endif
 
+// A store that later blocks of the same launch read: write-through at device scope, so that it is in memory once the
+// wavefront has waited for it and nobody has to write an XCD's L2 back.
+template <typename T> __device__ __forceinline__ void through_store(T* p, T v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// ... where FINISH says that there are such blocks
+template <bool FINISH, typename T> __device__ __forceinline__ void put_word(T* p, T v) {
+  if constexpr (FINISH) through_store(p, v);
+  else *p = v;
+}
+
+// ... and the load that goes with it.
+template <bool FINISH, typename T> __device__ __forceinline__ T get_word(const T* p) {
+  if constexpr (FINISH) return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  else return *p;
+}
+
 // Merge-path coordinate on diagonal `diag` of the merge of A = row_end[0..num_rows) (end offset of each
 // row) with B = 0..nnz-1.  Same search as the reference (include/merged_spmv_kernels.cuh:19-50):
 // the result x is the number of rows whose end offset is <= the number of non-zeros taken so far.
@@ -448,7 +465,9 @@ struct TileLds {
 // pointer would return the same two boundaries (boundary_from_split); the loads travel with the tile's own,
 // the verdict is part of the vote, and a tile whose boundaries are not confirmed returns true before
 // anything has been written: its block searches and comes back.
-template <class G, int BLOCK, int IPT, int EPL>
+// FINISH: another block of this launch folds the carries and partials (finish_launch): what it reads - the records and
+// the tile's first row, the only one a carry can belong to - is stored write-through.
+template <class G, int BLOCK, int IPT, int EPL, bool FINISH>
 __device__ __forceinline__ bool
 reduce_tile(const int tile, const int2 c0, const int2 c1, const Tiling& tl, const bool check, const int split0,
             const int split1, const int num_rows, const int* __restrict__ row_end, const int nnz,
@@ -757,12 +776,13 @@ reduce_tile(const int tile, const int2 c0, const int2 c1, const Tiling& tl, cons
           }
         }
         if (r < R) {
-          G::store_row(p, x0 + r, tot);
+          if (FINISH && r == 0) G::store_row_through(p, x0 + r, tot);
+          else G::store_row(p, x0 + r, tot);
         } else {  // r == R: the row still open at the end of the tile becomes the tile's carry
           const int row = x0 + r;
-          carry_row[tile] = (row < num_rows && len > 0) ? row : -1;
+          put_word<FINISH>(carry_row + tile, (row < num_rows && len > 0) ? row : -1);
 #pragma unroll
-          for (int c = 0; c < RED; ++c) carry_val[(size_t)tile * RED + c] = tot.v[c];
+          for (int c = 0; c < RED; ++c) put_word<FINISH>(carry_val + ((size_t)tile * RED + c), tot.v[c]);
         }
       };
       if (tid <= R) sum_row(tid, start1, len1, rowv);
@@ -966,9 +986,9 @@ reduce_tile(const int tile, const int2 c0, const int2 c1, const Tiling& tl, cons
       const int last_item = tile_items - 1;
       const bool open_empty = Z == 0 || (R > 0 && ((s_bits[last_item >> 5] >> (last_item & 31)) & 1u) != 0u);
       const int row = x0 + key;
-      carry_row[tile] = (row < num_rows && !open_empty) ? row : -1;
+      put_word<FINISH>(carry_row + tile, (row < num_rows && !open_empty) ? row : -1);
 #pragma unroll
-      for (int c = 0; c < RED; ++c) carry_val[(size_t)tile * RED + c] = run[c];
+      for (int c = 0; c < RED; ++c) put_word<FINISH>(carry_val + ((size_t)tile * RED + c), run[c]);
     }
     __syncthreads();
 
@@ -977,7 +997,8 @@ reduce_tile(const int tile, const int2 c0, const int2 c1, const Tiling& tl, cons
       Pack<V, RED> t;
 #pragma unroll
       for (int c = 0; c < RED; ++c) t.v[c] = s_out[c * TILE + i];
-      G::store_row(p, x0 + i, t);
+      if (FINISH && i == 0) G::store_row_through(p, x0 + i, t);
+      else G::store_row(p, x0 + i, t);
     }
   }
 
@@ -997,17 +1018,404 @@ reduce_tile(const int tile, const int2 c0, const int2 c1, const Tiling& tl, cons
       for (int c = 0; c < AGG; ++c) {
         V t = s_tile_agg[0][c];
         for (int w = 1; w < NW; ++w) t += s_tile_agg[w][c];
-        agg_partials[(size_t)tile * AGG + c] = t;
+        put_word<FINISH>(agg_partials + ((size_t)tile * AGG + c), t);
       }
     }
 #else  // tuning switch: one partial per wavefront, no barrier
     if (lane == WAVE - 1) {
 #pragma unroll
-      for (int c = 0; c < AGG; ++c) agg_partials[((size_t)tile * NW + wave) * AGG + c] = agg.v[c];
+      for (int c = 0; c < AGG; ++c) put_word<FINISH>(agg_partials + (((size_t)tile * NW + wave) * AGG + c), agg.v[c]);
     }
 #endif
   }
   return false;
+}
+
+// ----------------------------------------------------------------------------------------------
+// Fix-up: fold tile carries into their rows (tile order) and reduce the aggregator partials.
+//
+// Nothing here is about bytes: the work is a chain of memory latencies behind the reducer (an empty kernel costs 1.5 us
+// there), so it is written for few links.  A block takes BLOCK * PER tiles and loads all their carry rows and partials at
+// once, neighbouring lanes neighbouring tiles; a vote says what there is to do:
+//   no carry (most row-snapped launches)  nothing;
+//   no run of more than one tile          each carry and its row's current value are loaded together, added, stored;
+//   runs of tiles that carry into one row   a thread takes PER neighbouring tiles and sums the runs in them; where a run
+//       goes on from thread to thread, one block-wide segmented scan of the open sums (wave64 DPP scan, then a fold
+//       across the wavefronts in order) brings every thread what the run before it holds.  The thread of a run's last
+//       tile adds the total to the row.  A run that starts in the block and goes on beyond its tiles - a row of
+//       millions of non-zeros - is finished by the whole block: it walks the following tiles for as long as they carry
+//       into that row and adds them up in a fixed order; the blocks those tiles belong to see that their leading tiles
+//       continue an earlier run and leave them alone.
+// The same sums in the same order on every run, no floating-point atomics.
+//
+// Launches of at most 512 tiles are folded by 256 threads (the reducer's last block, or a kernel of one block), those of
+// a few thousand by one block of 1024.  Larger ones use blocks of 256 threads: a tile per thread where tiles carry, eight
+// on row-snapped launches.  With several blocks the one that draws the last ticket adds the blocks' aggregator sums, in
+// block order.  What it reads was stored write-through at device scope and had arrived before the ticket was drawn, so no
+// block has to write its XCD's L2 back: that release cost 15 us a launch, a kernel of its own for the sum 4.7.
+// Whole passes, against loads one tile after the other and the sum in a kernel of its own: spring-mass 100^3 25.9 ->
+// 25.0 us, rows of 18 to 81 entries (301 000 of them, float64) 43.5 -> 42.7, Poisson 256^3 308.6 -> 308.3.
+// ----------------------------------------------------------------------------------------------
+
+// Tiles [first, first + BLOCK * PER).  acc: receives the thread's share of the aggregators.
+template <class G, int BLOCK, int PARTS_PER_TILE, int PER, bool FINISH>
+__device__ __forceinline__ void
+fold_tiles(const typename G::Params& p, const int first, const int num_tiles, const int* __restrict__ carry_row,
+           const typename G::Value* __restrict__ carry_val, const typename G::Value* __restrict__ agg_partials,
+           Pack<typename G::Value, G::AGG_WIDTH>& acc) {
+  using V = typename G::Value;
+  constexpr int RED = G::RED_WIDTH, AGG = G::AGG_WIDTH;
+  constexpr int REDN = RED > 0 ? RED : 1;
+  constexpr int NW = BLOCK / WAVE;
+  constexpr int PARTS = AGG > 0 ? PARTS_PER_TILE * AGG : 1;
+  __shared__ int s_vote[NW];
+  __shared__ int s_key[NW];
+  __shared__ V s_val[NW][REDN];
+  __shared__ int s_lead_row, s_trail_row;
+  __shared__ V s_trail_val[REDN];
+  const int tid = threadIdx.x;
+  const int lane = tid & (WAVE - 1);
+  const int wave = tid / WAVE;
+  const int last = num_tiles - 1;
+  zero(acc);
+  int vote = 0;
+  int lead_row = -1;  // the row of a run an earlier block finishes
+  {
+    // neighbouring lanes take neighbouring tiles here: everything in whole lines
+    int row[PER], before[PER], after[PER];
+    V part[PER][PARTS];
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const int t = min(first + i * BLOCK + tid, last);
+      row[i] = get_word<FINISH>(carry_row + t);
+      before[i] = get_word<FINISH>(carry_row + max(t - 1, 0));
+      after[i] = get_word<FINISH>(carry_row + min(t + 1, last));
+#pragma unroll
+      for (int c = 0; c < (AGG > 0 ? PARTS : 0); ++c) part[i][c] = get_word<FINISH>(agg_partials + ((size_t)t * PARTS + c));
+    }
+    bool any = false, runs = false;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const int t = first + i * BLOCK + tid;
+      if (t > last) row[i] = -1;
+      if (i == 0 && tid == 0) s_lead_row = t > 0 && row[0] >= 0 && before[0] == row[0] ? row[0] : -1;
+      any |= row[i] >= 0;
+      runs |= row[i] >= 0 && ((t > 0 && before[i] == row[i]) || (t < last && after[i] == row[i]));
+#pragma unroll
+      for (int c = 0; c < (AGG > 0 ? PARTS : 0); ++c) acc.v[c % (AGG > 0 ? AGG : 1)] += t <= last ? part[i][c] : V(0);
+    }
+    if constexpr (RED > 0) {
+      const int mine = (__builtin_amdgcn_ballot_w64(any) != 0ull ? 1 : 0) | (__builtin_amdgcn_ballot_w64(runs) != 0ull ? 2 : 0);
+      if (lane == 0) s_vote[wave] = mine;
+      if (tid == 0) s_trail_row = -1;
+      __syncthreads();
+#pragma unroll
+      for (int w = 0; w < NW; ++w) vote |= s_vote[w];
+      lead_row = s_lead_row;
+      if (vote == 1) {  // no run of more than one tile: every carry and its row's value loaded together, added, stored
+        constexpr int WORDS = RED * (int)(sizeof(V) / 4);
+        constexpr int TOGETHER = WORDS * PER <= 16 ? PER : (WORDS >= 16 ? 1 : 16 / WORDS);  // within 32 registers
+#pragma unroll
+        for (int i0 = 0; i0 < PER; i0 += TOGETHER) {
+          Pack<V, RED> sum[TOGETHER], now[TOGETHER];
+#pragma unroll
+          for (int k = 0; k < TOGETHER; ++k) {
+            const int i = i0 + k < PER ? i0 + k : PER - 1;
+            const int t = min(first + i * BLOCK + tid, last);
+#pragma unroll
+            for (int c = 0; c < RED; ++c) sum[k].v[c] = get_word<FINISH>(carry_val + ((size_t)t * RED + c));
+            G::current_row(p, max(row[i], 0), now[k]);
+          }
+#pragma unroll
+          for (int k = 0; k < TOGETHER; ++k) {
+            const int i = i0 + k < PER ? i0 + k : PER - 1;
+            if (i0 + k < PER && row[i] >= 0) {
+#pragma unroll
+              for (int c = 0; c < RED; ++c) now[k].v[c] += sum[k].v[c];
+              G::store_row(p, row[i], now[k]);
+            }
+          }
+        }
+      }
+    }
+  }
+  if constexpr (RED > 0) {
+    if ((vote & 2) == 0) return;
+    // runs: a thread takes PER neighbouring tiles
+    const int t0 = first + tid * PER;
+    int row[PER + 1];  // of the thread's tiles, and of the one after them
+#pragma unroll
+    for (int i = 0; i <= PER; ++i) {
+      const int r = get_word<FINISH>(carry_row + min(t0 + i, last));
+      row[i] = t0 + i <= last ? r : -1;
+    }
+    // the carries' values: kept in registers where they fit, else read again from memory where they are needed
+    constexpr bool KEEP = RED * PER * (int)(sizeof(V) / 4) <= 32;
+    V kept[KEEP ? PER : 1][REDN];
+    auto value = [&](const int i, const int c) {
+      return KEEP ? kept[KEEP ? i : 0][c] : get_word<FINISH>(carry_val + ((size_t)min(t0 + i, last) * RED + c));
+    };
+    if constexpr (KEEP) {
+#pragma unroll
+      for (int i = 0; i < PER; ++i) {
+#pragma unroll
+        for (int c = 0; c < RED; ++c) kept[i][c] = get_word<FINISH>(carry_val + ((size_t)min(t0 + i, last) * RED + c));
+      }
+    }
+    // adds tile i to the sum of its run, which starts afresh where the row changes
+    auto add_tile = [&](const int i, V (&sum)[REDN]) {
+      const bool fresh = i > 0 && row[i] != row[i > 0 ? i - 1 : 0];
+#pragma unroll
+      for (int c = 0; c < RED; ++c) {
+        const V v = value(i, c);
+        sum[c] = (fresh ? V(0) : sum[c]) + (row[i] >= 0 ? v : V(0));
+      }
+    };
+    V in[REDN];  // what the threads before this one hold of the run its first tile continues
+#pragma unroll
+    for (int c = 0; c < RED; ++c) in[c] = V(0);
+    {
+      V open[REDN];
+#pragma unroll
+      for (int c = 0; c < RED; ++c) open[c] = V(0);
+#pragma unroll
+      for (int i = 0; i < PER; ++i) add_tile(i, open);
+      const int key = row[PER - 1] >= 0 && row[PER] == row[PER - 1] ? row[PER] : -1;  // the run open behind the thread
+#pragma unroll
+      for (int c = 0; c < RED; ++c) open[c] = key >= 0 ? open[c] : V(0);
+      wave_segmented_inclusive_sum<V, REDN>(key, open);
+      int in_key = wave_shift_up1<int>(key, -1);
+#pragma unroll
+      for (int c = 0; c < RED; ++c) in[c] = wave_shift_up1<V>(open[c], V(0));
+      if (lane == WAVE - 1) {
+        s_key[wave] = key;
+#pragma unroll
+        for (int c = 0; c < RED; ++c) s_val[wave][c] = open[c];
+      }
+      __syncthreads();
+      int pk = -1;
+      V pv[REDN];
+#pragma unroll
+      for (int c = 0; c < RED; ++c) pv[c] = V(0);
+#pragma unroll
+      for (int w = 0; w < NW - 1; ++w) {
+        if (w < wave) {
+          const int k = s_key[w];
+#pragma unroll
+          for (int c = 0; c < RED; ++c) pv[c] = (k == pk) ? static_cast<V>(pv[c] + s_val[w][c]) : s_val[w][c];
+          pk = k;
+        }
+      }
+      if (wave > 0 && lane == 0) {
+        in_key = pk;
+#pragma unroll
+        for (int c = 0; c < RED; ++c) in[c] = pv[c];
+      } else if (wave > 0 && in_key == pk) {
+#pragma unroll
+        for (int c = 0; c < RED; ++c) in[c] += pv[c];
+      }
+      if (tid == BLOCK - 1 && key >= 0 && key != lead_row) {  // goes on beyond the block's tiles
+        s_trail_row = key;
+#pragma unroll
+        for (int c = 0; c < RED; ++c) s_trail_val[c] = open[c] + (wave > 0 && key == pk ? pv[c] : V(0));
+      }
+#pragma unroll
+      for (int c = 0; c < RED; ++c) in[c] = in_key >= 0 && in_key == row[0] ? in[c] : V(0);
+    }
+    // the runs that end in the thread's tiles: current values of their rows loaded together, then added and stored
+    constexpr int WORDS = RED * (int)(sizeof(V) / 4);
+    constexpr int TOGETHER = WORDS * PER <= 32 ? PER : (WORDS >= 32 ? 1 : 32 / WORDS);
+#pragma unroll
+    for (int i0 = 0; i0 < PER; i0 += TOGETHER) {
+      Pack<V, RED> now[TOGETHER];
+#pragma unroll
+      for (int k = 0; k < TOGETHER; ++k) {
+        if (i0 + k < PER) G::current_row(p, max(row[i0 + k < PER ? i0 + k : 0], 0), now[k]);
+      }
+#pragma unroll
+      for (int k = 0; k < TOGETHER; ++k) {
+        const int i = i0 + k;
+        if (i < PER) {
+          add_tile(i, in);
+          if (row[i] >= 0 && row[i + 1] != row[i] && row[i] != lead_row) {
+#pragma unroll
+            for (int c = 0; c < RED; ++c) now[k].v[c] += in[c];
+            G::store_row(p, row[i], now[k]);
+          }
+        }
+      }
+    }
+    __syncthreads();
+    const int trail_row = s_trail_row;
+    if (trail_row < 0) return;  // uniform
+    V ext[REDN];
+#pragma unroll
+    for (int c = 0; c < RED; ++c) ext[c] = V(0);
+    // EXT_STEP * BLOCK tiles per vote, all their loads in flight together (the values are fetched whether or not the
+    // tile belongs to the run: a load under the test would wait for the row first)
+    constexpr int EXT_STEP = 4;
+    for (int base = first + BLOCK * PER; base < num_tiles; base += EXT_STEP * BLOCK) {
+      int urow[EXT_STEP];
+      V uval[EXT_STEP][REDN];
+#pragma unroll
+      for (int k = 0; k < EXT_STEP; ++k) {
+        const int u = min(base + k * BLOCK + tid, last);
+        urow[k] = get_word<FINISH>(carry_row + u);
+#pragma unroll
+        for (int c = 0; c < RED; ++c) uval[k][c] = get_word<FINISH>(carry_val + ((size_t)u * RED + c));
+      }
+      bool all_same = true;
+#pragma unroll
+      for (int k = 0; k < EXT_STEP; ++k) {
+        const bool same = base + k * BLOCK + tid < num_tiles && urow[k] == trail_row;
+        all_same &= same;
+        if (same) {
+#pragma unroll
+          for (int c = 0; c < RED; ++c) ext[c] += uval[k][c];
+        }
+      }
+      if (!__syncthreads_and(all_same ? 1 : 0)) break;  // the run is contiguous: a mismatch ends it
+    }
+    wave_sum_to_last_lane<V, REDN>(ext);
+    __syncthreads();  // s_val is free again
+    if (lane == WAVE - 1) {
+#pragma unroll
+      for (int c = 0; c < RED; ++c) s_val[wave][c] = ext[c];
+    }
+    __syncthreads();
+    if (tid == 0) {
+      Pack<V, RED> sum;
+#pragma unroll
+      for (int c = 0; c < RED; ++c) {
+        V x = s_trail_val[c];
+#pragma unroll
+        for (int w = 0; w < NW; ++w) x += s_val[w][c];
+        sum.v[c] = x;
+      }
+      G::add_row(p, trail_row, sum);
+    }
+  }
+}
+
+// ... `per` tiles per thread, uniform over the launch, at most MAX_PER (2 or 8) of them
+template <class G, int BLOCK, int PARTS_PER_TILE, int MAX_PER, bool FINISH>
+__device__ __forceinline__ void
+fixup_tiles(const typename G::Params& p, const int block, const int num_tiles, const int per,
+            const int* __restrict__ carry_row, const typename G::Value* __restrict__ carry_val,
+            const typename G::Value* __restrict__ agg_partials, Pack<typename G::Value, G::AGG_WIDTH>& acc) {
+  auto fold = [&](auto per_tag) {
+    constexpr int PER = decltype(per_tag)::value;
+    fold_tiles<G, BLOCK, PARTS_PER_TILE, PER, FINISH>(p, block * BLOCK * PER, num_tiles, carry_row, carry_val, agg_partials, acc);
+  };
+  if (per == 1) fold(std::integral_constant<int, 1>{});
+  else if (MAX_PER == 2 || per == 2) fold(std::integral_constant<int, 2>{});
+  else if (per <= 4) fold(std::integral_constant<int, MAX_PER < 4 ? MAX_PER : 4>{});
+  else fold(std::integral_constant<int, MAX_PER>{});
+}
+
+// The block's sum of the threads' shares, in a fixed order; valid in every thread.
+template <typename V, int AGG, int BLOCK>
+__device__ __forceinline__ Pack<V, AGG> block_total(Pack<V, AGG> share) {
+  constexpr int NW = BLOCK / WAVE;
+  __shared__ V s_wave_agg[NW][AGG];
+  const int tid = threadIdx.x;
+  wave_sum_to_last_lane<V, AGG>(share.v);
+  __syncthreads();  // a block may add up twice
+  if ((tid & (WAVE - 1)) == WAVE - 1) {
+#pragma unroll
+    for (int c = 0; c < AGG; ++c) s_wave_agg[tid / WAVE][c] = share.v[c];
+  }
+  __syncthreads();
+  Pack<V, AGG> total;
+#pragma unroll
+  for (int c = 0; c < AGG; ++c) {
+    V s = s_wave_agg[0][c];
+#pragma unroll
+    for (int w = 1; w < NW; ++w) s += s_wave_agg[w][c];
+    total.v[c] = s;
+  }
+  return total;
+}
+
+// `count` partial vectors added by the block in a fixed order, BLOCK * 4 loads at a time; valid in every thread.
+template <class G, int BLOCK, bool FINISH>
+__device__ __forceinline__ Pack<typename G::Value, G::AGG_WIDTH>
+sum_partials(const typename G::Value* __restrict__ partials, const int count) {
+  using V = typename G::Value;
+  constexpr int AGG = G::AGG_WIDTH, BATCH = 4;
+  Pack<V, AGG> acc;
+  zero(acc);
+  for (int j0 = threadIdx.x; j0 < count; j0 += BATCH * BLOCK) {
+    V v[BATCH][AGG];
+#pragma unroll
+    for (int k = 0; k < BATCH; ++k) {
+      const int j = min(j0 + k * BLOCK, count - 1);
+#pragma unroll
+      for (int c = 0; c < AGG; ++c) v[k][c] = get_word<FINISH>(partials + ((size_t)j * AGG + c));
+    }
+#pragma unroll
+    for (int k = 0; k < BATCH; ++k) {
+#pragma unroll
+      for (int c = 0; c < AGG; ++c) acc.v[c] += j0 + k * BLOCK < count ? v[k][c] : V(0);
+    }
+  }
+  return block_total<V, AGG, BLOCK>(acc);
+}
+
+// Is this block (number `block` of `blocks`) the last of the launch?  Its through_store()s are visible to the block that
+// is.  Same-address atomics of different XCDs take 12 ns each, so blocks are counted in groups of 32, the groups in one
+// more counter, each on a 128-byte line of its own; the last to arrive leaves every counter at zero for the next launch.
+constexpr int FINISH_GROUP = 32;
+constexpr int FINISH_PER = 2;  // tiles per thread of the block that finishes, at most
+__device__ __forceinline__ bool last_block(unsigned* counters, const int block, const int blocks) {
+  __shared__ int s_last;
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // every wavefront: its stores have arrived
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    auto arrive = [](unsigned* counter, const int of) {
+      if (__hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != (unsigned)of - 1u) return false;
+      through_store(counter, 0u);
+      return true;
+    };
+    const int group = block / FINISH_GROUP;
+    s_last = arrive(counters + 32 * (1 + group), min(FINISH_GROUP, blocks - group * FINISH_GROUP)) &&
+             arrive(counters, (blocks + FINISH_GROUP - 1) / FINISH_GROUP);
+  }
+  __syncthreads();
+  if (s_last == 0) return false;
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+  return true;
+}
+
+template <class G, int BLOCK, int PARTS_PER_TILE>
+__global__ void __launch_bounds__(BLOCK)
+fixup_kernel(const int* __restrict__ carry_row, const typename G::Value* __restrict__ agg_partials,
+             const typename G::Value* __restrict__ carry_val, const int num_tiles, const int per,
+             typename G::Value* __restrict__ block_partials, unsigned* __restrict__ ticket, const typename G::Params p) {
+  using V = typename G::Value;
+  constexpr int AGG = G::AGG_WIDTH;
+  Pack<V, AGG> acc;
+  fixup_tiles<G, BLOCK, PARTS_PER_TILE, 8, false>(p, (int)blockIdx.x, num_tiles, per, carry_row, carry_val, agg_partials, acc);
+  if constexpr (AGG > 0) {
+    __shared__ int s_is_last;
+    const Pack<V, AGG> total = block_total<V, AGG, BLOCK>(acc);
+    if (gridDim.x == 1) {
+      if (threadIdx.x == 0) G::store_agg(p, total);
+      return;
+    }
+    if (threadIdx.x == 0) {
+#pragma unroll
+      for (int c = 0; c < AGG; ++c) through_store(&block_partials[(size_t)blockIdx.x * AGG + c], total.v[c]);
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the stores above have arrived before the ticket is drawn
+      s_is_last = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1 ? 1 : 0;
+    }
+    __syncthreads();
+    if (s_is_last) {
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+      const Pack<V, AGG> all = sum_partials<G, BLOCK, true>(block_partials, (int)gridDim.x);
+      if (threadIdx.x == 0) G::store_agg(p, all);
+    }
+  }
 }
 
 // Where a reducer block takes its tile's two boundaries from.
@@ -1033,16 +1441,33 @@ enum TileSource : int {
 // With FLEX_TUNE_PERSISTENT (tuning switch) a launch has at most that many blocks per CU; each walks
 // tiles blockIdx.x, blockIdx.x + gridDim.x, ... and reads the coordinates of its next tile while it
 // works on the current one.
-template <class G, int BLOCK, int IPT, int EPL>
+//
+// FINISH (launches of at most FINISH_MAX_TILES tiles whose caller keeps counters): the last block to finish does the
+// fix-up, and the launch is one kernel.  A kernel costs the host 2.7 to 4 us to issue, more than these launches run for.
+template <class G, int BLOCK, int IPT, int EPL, bool FINISH>
 __global__ void __launch_bounds__(BLOCK)
 reduce_kernel(int2* coords, int* splits, const int* __restrict__ row_end, const int source, const int xcd_shift,
               const int tiles, const int num_rows, const int nnz, const int nominal, const int snap_slack,
               const int snap_mask, const int row_group, const typename G::Params p, int* __restrict__ carry_row,
               typename G::Value* __restrict__ carry_val, typename G::Value* __restrict__ agg_partials,
-              unsigned* __restrict__ ticket) {
+              unsigned* __restrict__ counters) {
   const Tiling tl{tiles, nominal, snap_slack, snap_mask, xcd_shift, row_group};
   const int num_tiles = tl.num_tiles;
-  if (G::AGG_WIDTH > 0 && blockIdx.x == 0 && threadIdx.x == 0) *ticket = 0u;  // for the fixup_kernel of this launch
+  // (without FINISH: the ticket of this launch's fixup_kernel)
+  if (!FINISH && G::AGG_WIDTH > 0 && blockIdx.x == 0 && threadIdx.x == 0) *counters = 0u;
+  auto finish = [&](const int tile) {
+    if constexpr (FINISH) {
+      if (!last_block(counters, tile, tl.num_tiles)) return;
+      constexpr int AGG = G::AGG_WIDTH;
+      Pack<typename G::Value, AGG> acc;
+      fixup_tiles<G, BLOCK, partials_per_tile<BLOCK>(), FINISH_PER, true>(p, 0, tl.num_tiles, (tl.num_tiles + BLOCK - 1) / BLOCK,
+                                                                         carry_row, carry_val, agg_partials, acc);
+      if constexpr (AGG > 0) {
+        const Pack<typename G::Value, AGG> total = block_total<typename G::Value, AGG, BLOCK>(acc);
+        if (threadIdx.x == 0) G::store_agg(p, total);
+      }
+    }
+  };
 #ifdef FLEX_TUNE_PERSISTENT
   int tile = blockIdx.x;
   if (tile >= num_tiles) return;
@@ -1055,7 +1480,7 @@ reduce_kernel(int2* coords, int* splits, const int* __restrict__ row_end, const 
       n0 = coords[next];
       n1 = coords[next + 1];
     }
-    reduce_tile<G, BLOCK, IPT, EPL>(tile, c0, c1, tl, false, 0, 0, num_rows, row_end, nnz, p, carry_row, carry_val, agg_partials);
+    reduce_tile<G, BLOCK, IPT, EPL, FINISH>(tile, c0, c1, tl, false, 0, 0, num_rows, row_end, nnz, p, carry_row, carry_val, agg_partials);
     if (!more) break;
     __syncthreads();  // the tile's LDS is free again
     tile = next;
@@ -1097,9 +1522,12 @@ reduce_kernel(int2* coords, int* splits, const int* __restrict__ row_end, const 
   // derived from the thread id in registers through the whole tile: 12 scalar spills and up to 17 more
   // vector registers, 3 % of the kernel on the 3-D stencil).
   if (have) {
-    const bool refused = reduce_tile<G, BLOCK, IPT, EPL>(tile, c0, c1, tl, check, split0, split1, num_rows, row_end, nnz,
+    const bool refused = reduce_tile<G, BLOCK, IPT, EPL, FINISH>(tile, c0, c1, tl, check, split0, split1, num_rows, row_end, nnz,
                                                          p, carry_row, carry_val, agg_partials);
-    if (!refused) return;
+    if (!refused) {
+      finish(tile);
+      return;
+    }
     __syncthreads();  // every thread has read the verdict; the tile's LDS is free again
   }
   {
@@ -1139,8 +1567,9 @@ reduce_kernel(int2* coords, int* splits, const int* __restrict__ row_end, const 
         splits[num_tiles] = s_split[1];
       }
     }
-    reduce_tile<G, BLOCK, IPT, EPL>(tile, c0, c1, tl, false, 0, 0, num_rows, row_end, nnz, p, carry_row, carry_val,
-                                    agg_partials);
+    reduce_tile<G, BLOCK, IPT, EPL, FINISH>(tile, c0, c1, tl, false, 0, 0, num_rows, row_end, nnz, p, carry_row, carry_val,
+                                            agg_partials);
+    finish(tile);
   }
 #endif
 }
@@ -1148,15 +1577,13 @@ reduce_kernel(int2* coords, int* splits, const int* __restrict__ row_end, const 
 // ----------------------------------------------------------------------------------------------
 // Flat kernel (aggregator and map-only graphs): tiles are plain edge ranges, no row structure.
 // ----------------------------------------------------------------------------------------------
-template <class G, int BLOCK, int IPT>
+template <class G, int BLOCK, int IPT, bool FINISH>
 __global__ void __launch_bounds__(BLOCK)
 flat_kernel(const typename G::Params p, const int nnz, const int num_tiles,
-            typename G::Value* __restrict__ agg_partials) {
+            typename G::Value* __restrict__ agg_partials, unsigned* __restrict__ counters) {
   using V = typename G::Value;
   constexpr int TILE = BLOCK * IPT;
-  constexpr int NW = BLOCK / WAVE;
   constexpr int AGG = G::AGG_WIDTH;
-  __shared__ V s_wave_agg[NW][AGG > 0 ? AGG : 1];
 
   const int tid = threadIdx.x;
   Pack<V, AGG> agg;
@@ -1184,298 +1611,16 @@ flat_kernel(const typename G::Params p, const int nnz, const int num_tiles,
     }
   }
   if constexpr (AGG > 0) {
-    wave_sum_to_last_lane<V, AGG>(agg.v);
-    if ((tid & (WAVE - 1)) == WAVE - 1) {
-#pragma unroll
-      for (int c = 0; c < AGG; ++c) s_wave_agg[tid / WAVE][c] = agg.v[c];
-    }
-    __syncthreads();
+    const Pack<V, AGG> total = block_total<V, AGG, BLOCK>(agg);
     if (tid == 0) {
 #pragma unroll
-      for (int c = 0; c < AGG; ++c) {
-        V s = s_wave_agg[0][c];
-        for (int w = 1; w < NW; ++w) s += s_wave_agg[w][c];
-        agg_partials[(size_t)blockIdx.x * AGG + c] = s;
-      }
+      for (int c = 0; c < AGG; ++c) put_word<FINISH>(agg_partials + ((size_t)blockIdx.x * AGG + c), total.v[c]);
     }
-  }
-}
-
-// ----------------------------------------------------------------------------------------------
-// Fix-up: fold tile carries into their rows (tile order) and reduce the aggregator partials.
-//
-// Nothing here is about bytes: the kernel is a chain of memory latencies behind the reducer (an empty kernel costs
-// 1.5 us there), so it is written for few links.  A block takes BLOCK * per tiles, `per` a thread, and loads all their
-// carry rows and partials at once; a vote says what there is to do:
-//   no carry (row-snapped launches)       nothing;
-//   no run of more than one tile          each carry and its row's current value are loaded together, added, stored;
-//   a run of tiles that carry into one row  the block walks its tiles in chunks of BLOCK and sums the run by a segmented
-//       scan (wave64 DPP scan, then a fold across the wavefronts in order); the thread of the run's last tile adds the
-//       total to the row.  A run that starts in the chunk and goes on beyond it - a row of millions of non-zeros - is
-//       finished by the whole block: it walks the following tiles BLOCK at a time for as long as they carry into that
-//       row and adds them up in a fixed order; the chunks those tiles belong to see that their leading tiles continue an
-//       earlier run and leave them alone.
-// The same sums in the same order on every run, no floating-point atomics.
-//
-// Launches of a few thousand tiles use one block of 1024 threads.  Larger ones use blocks of 256 threads: a tile per
-// thread where tiles carry (runs are common there, and blocks walk them side by side), eight per thread on row-snapped
-// launches.  With several blocks the one that draws the last ticket adds the blocks' aggregator sums, in block order.
-// What it reads was stored write-through at device scope and had arrived before the ticket was drawn, so no block
-// has to write its XCD's L2 back: that release cost 15 us a launch, a kernel of its own for the sum 4.7.
-// Whole passes, against loads one tile after the other and the sum in a kernel of its own: spring-mass 100^3 25.9 ->
-// 25.0 us, rows of 18 to 81 entries (301 000 of them, float64) 43.5 -> 42.7, Poisson 256^3 308.6 -> 308.3.
-// ----------------------------------------------------------------------------------------------
-
-// One pass over the block's tiles; returns whether the block has runs to walk.  acc: the thread's share of the
-// aggregators.
-template <class G, int BLOCK, int PARTS_PER_TILE, int PER>
-__device__ __forceinline__ bool
-fold_single_carries(const typename G::Params& p, const int first, const int num_tiles, const int* __restrict__ carry_row,
-                    const typename G::Value* __restrict__ carry_val, const typename G::Value* __restrict__ agg_partials,
-                    int* s_vote, Pack<typename G::Value, G::AGG_WIDTH>& acc) {
-  using V = typename G::Value;
-  constexpr int RED = G::RED_WIDTH, AGG = G::AGG_WIDTH;
-  constexpr int NW = BLOCK / WAVE;
-  constexpr int PARTS = AGG > 0 ? PARTS_PER_TILE * AGG : 1;
-  const int tid = threadIdx.x;
-  const int last = num_tiles - 1;
-  int row[PER], before[PER], after[PER];
-  V part[PER][PARTS];
-#pragma unroll
-  for (int i = 0; i < PER; ++i) {
-    const int t = min(first + i * BLOCK + tid, last);
-    row[i] = carry_row[t];
-    before[i] = carry_row[max(t - 1, 0)];
-    after[i] = carry_row[min(t + 1, last)];
-#pragma unroll
-    for (int c = 0; c < (AGG > 0 ? PARTS : 0); ++c) part[i][c] = agg_partials[(size_t)t * PARTS + c];
-  }
-  bool any = false, runs = false;
-#pragma unroll
-  for (int i = 0; i < PER; ++i) {
-    const int t = first + i * BLOCK + tid;
-    if (t > last) row[i] = -1;
-    any |= row[i] >= 0;
-    runs |= row[i] >= 0 && t < last && after[i] == row[i];
-    if (t > 0 && before[i] == row[i]) row[i] = -1;  // belongs to a run whose first tile another thread (or block) has
-#pragma unroll
-    for (int c = 0; c < (AGG > 0 ? PARTS : 0); ++c) acc.v[c % (AGG > 0 ? AGG : 1)] += t <= last ? part[i][c] : V(0);
-  }
-  if constexpr (RED > 0) {
-    const int mine = (__builtin_amdgcn_ballot_w64(any) != 0ull ? 1 : 0) | (__builtin_amdgcn_ballot_w64(runs) != 0ull ? 2 : 0);
-    if ((tid & (WAVE - 1)) == 0) s_vote[tid / WAVE] = mine;
-    __syncthreads();
-    int vote = 0;
-#pragma unroll
-    for (int w = 0; w < NW; ++w) vote |= s_vote[w];
-    if (vote == 0) return false;
-    if ((vote & 2) != 0) return true;
-    constexpr int WORDS = RED * (int)(sizeof(V) / 4);
-    constexpr int TOGETHER = WORDS * PER <= 16 ? PER : (WORDS >= 16 ? 1 : 16 / WORDS);  // within 32 registers
-    for (int i0 = 0; i0 < PER; i0 += TOGETHER) {
-      Pack<V, RED> sum[TOGETHER], now[TOGETHER];
-#pragma unroll
-      for (int k = 0; k < TOGETHER; ++k) {
-        const int i = min(i0 + k, PER - 1);
-        const int t = min(first + i * BLOCK + tid, last);
-#pragma unroll
-        for (int c = 0; c < RED; ++c) sum[k].v[c] = carry_val[(size_t)t * RED + c];
-        G::current_row(p, max(row[i], 0), now[k]);
+    if constexpr (FINISH) {
+      if (last_block(counters, blockIdx.x, gridDim.x)) {
+        const Pack<V, AGG> all = sum_partials<G, BLOCK, true>(agg_partials, (int)gridDim.x);
+        if (tid == 0) G::store_agg(p, all);
       }
-#pragma unroll
-      for (int k = 0; k < TOGETHER; ++k) {
-        const int i = i0 + k;
-        if (i < PER && row[i < PER ? i : 0] >= 0) {
-#pragma unroll
-          for (int c = 0; c < RED; ++c) now[k].v[c] += sum[k].v[c];
-          G::store_row(p, row[i < PER ? i : 0], now[k]);
-        }
-      }
-    }
-  }
-  return false;
-}
-
-template <class G, int BLOCK, int PARTS_PER_TILE>
-__global__ void __launch_bounds__(BLOCK)
-fixup_kernel(const int* __restrict__ carry_row, const typename G::Value* __restrict__ agg_partials,
-             const typename G::Value* __restrict__ carry_val, const int num_tiles, const int per,
-             typename G::Value* __restrict__ block_partials, unsigned* __restrict__ ticket, const typename G::Params p) {
-  using V = typename G::Value;
-  constexpr int RED = G::RED_WIDTH, AGG = G::AGG_WIDTH;
-  constexpr int REDN = RED > 0 ? RED : 1;
-  constexpr int NW = BLOCK / WAVE;
-  const int tid = threadIdx.x;
-  const int lane = tid & (WAVE - 1);
-  const int wave = tid / WAVE;
-  __shared__ int s_vote[NW];
-  __shared__ int s_key[NW];
-  __shared__ V s_val[NW][REDN];
-  __shared__ int s_trail_row;
-  __shared__ V s_trail_val[REDN];
-  Pack<V, AGG> acc;
-  zero(acc);
-  const int first = (int)blockIdx.x * BLOCK * per;
-  auto fold = [&](auto per_tag) {
-    return fold_single_carries<G, BLOCK, PARTS_PER_TILE, decltype(per_tag)::value>(p, first, num_tiles, carry_row, carry_val,
-                                                                                   agg_partials, s_vote, acc);
-  };
-  const bool runs = per == 1 ? fold(std::integral_constant<int, 1>{})   // uniform over the launch
-                    : per == 2 ? fold(std::integral_constant<int, 2>{})
-                    : per <= 4 ? fold(std::integral_constant<int, 4>{})
-                               : fold(std::integral_constant<int, 8>{});
-  if constexpr (RED > 0) {
-    for (int chunk = first; runs && chunk < min(first + BLOCK * per, num_tiles); chunk += BLOCK) {
-      const int t = chunk + tid;
-      const bool valid = t < num_tiles;
-      const int row = valid ? carry_row[t] : -1;
-      const int next_row = (valid && t + 1 < num_tiles) ? carry_row[t + 1] : -2;
-      V run[REDN];
-#pragma unroll
-      for (int c = 0; c < RED; ++c) run[c] = (row >= 0) ? carry_val[(size_t)t * RED + c] : V(0);
-      // does the chunk start inside a run that an earlier chunk owns?
-      const int chunk_first_row = carry_row[chunk];
-      const bool leading_continues = chunk > 0 && chunk_first_row >= 0 && carry_row[chunk - 1] == chunk_first_row;
-      // segmented inclusive sums over the chunk, keyed by row (equal rows are contiguous)
-      wave_segmented_inclusive_sum<V, REDN>(row, run);
-      if (tid == 0) s_trail_row = -1;
-      if (lane == WAVE - 1) {
-        s_key[wave] = row;
-#pragma unroll
-        for (int c = 0; c < RED; ++c) s_val[wave][c] = run[c];
-      }
-      __syncthreads();
-      {
-        int pk = -3;
-        V pv[REDN];
-#pragma unroll
-        for (int c = 0; c < RED; ++c) pv[c] = V(0);
-#pragma unroll
-        for (int w = 0; w < NW - 1; ++w) {
-          if (w < wave) {
-            const int k = s_key[w];
-#pragma unroll
-            for (int c = 0; c < RED; ++c) pv[c] = (k == pk) ? static_cast<V>(pv[c] + s_val[w][c]) : s_val[w][c];
-            pk = k;
-          }
-        }
-        if (wave > 0 && row >= 0 && row == pk) {  // my run began in an earlier wavefront of this chunk
-#pragma unroll
-          for (int c = 0; c < RED; ++c) run[c] += pv[c];
-        }
-      }
-      const bool mine = row >= 0 && !(leading_continues && row == chunk_first_row);
-      const bool part_end = next_row != row || tid == BLOCK - 1;  // last tile of the run inside this chunk
-      if (mine && part_end) {
-        if (next_row != row) {  // the run ends here
-          Pack<V, RED> sum;
-#pragma unroll
-          for (int c = 0; c < RED; ++c) sum.v[c] = run[c];
-          G::add_row(p, row, sum);
-        } else {  // it goes on in the following chunks: the block finishes it together
-          s_trail_row = row;
-#pragma unroll
-          for (int c = 0; c < RED; ++c) s_trail_val[c] = run[c];
-        }
-      }
-      __syncthreads();
-      const int trail_row = s_trail_row;
-      if (trail_row >= 0) {  // uniform
-        V ext[REDN];
-#pragma unroll
-        for (int c = 0; c < RED; ++c) ext[c] = V(0);
-        // EXT_STEP chunks per vote, all their loads in flight together (the values are fetched whether or
-        // not the tile belongs to the run: a load under the test would wait for the row first)
-        constexpr int EXT_STEP = 4;
-        const int last_tile = num_tiles - 1;
-        for (int base = chunk + BLOCK; base < num_tiles; base += EXT_STEP * BLOCK) {
-          int urow[EXT_STEP];
-          V uval[EXT_STEP][REDN];
-#pragma unroll
-          for (int k = 0; k < EXT_STEP; ++k) {
-            const int u = min(base + k * BLOCK + tid, last_tile);
-            urow[k] = carry_row[u];
-#pragma unroll
-            for (int c = 0; c < RED; ++c) uval[k][c] = carry_val[(size_t)u * RED + c];
-          }
-          bool all_same = true;
-#pragma unroll
-          for (int k = 0; k < EXT_STEP; ++k) {
-            const bool same = base + k * BLOCK + tid < num_tiles && urow[k] == trail_row;
-            all_same &= same;
-            if (same) {
-#pragma unroll
-              for (int c = 0; c < RED; ++c) ext[c] += uval[k][c];
-            }
-          }
-          if (!__syncthreads_and(all_same ? 1 : 0)) break;  // the run is contiguous: a mismatch ends it
-        }
-        wave_sum_to_last_lane<V, REDN>(ext);
-        __syncthreads();  // s_val is free again
-        if (lane == WAVE - 1) {
-#pragma unroll
-          for (int c = 0; c < RED; ++c) s_val[wave][c] = ext[c];
-        }
-        __syncthreads();
-        if (tid == 0) {
-          Pack<V, RED> sum;
-#pragma unroll
-          for (int c = 0; c < RED; ++c) {
-            V x = s_trail_val[c];
-#pragma unroll
-            for (int w = 0; w < NW; ++w) x += s_val[w][c];
-            sum.v[c] = x;
-          }
-          G::add_row(p, trail_row, sum);
-        }
-      }
-      __syncthreads();  // before the next chunk reuses the shared arrays
-    }
-  }
-  if constexpr (AGG > 0) {
-    __shared__ V s_wave_agg[NW][AGG];
-    __shared__ int s_is_last;
-    auto block_total = [&](Pack<V, AGG>& share) {  // the block's sum, in thread 0
-      wave_sum_to_last_lane<V, AGG>(share.v);
-      if (lane == WAVE - 1) {
-#pragma unroll
-        for (int c = 0; c < AGG; ++c) s_wave_agg[wave][c] = share.v[c];
-      }
-      __syncthreads();
-      Pack<V, AGG> total;
-#pragma unroll
-      for (int c = 0; c < AGG; ++c) {
-        V s = s_wave_agg[0][c];
-#pragma unroll
-        for (int w = 1; w < NW; ++w) s += s_wave_agg[w][c];
-        total.v[c] = s;
-      }
-      return total;
-    };
-    const Pack<V, AGG> total = block_total(acc);
-    if (gridDim.x == 1) {
-      if (tid == 0) G::store_agg(p, total);
-      return;
-    }
-    if (tid == 0) {
-#pragma unroll
-      for (int c = 0; c < AGG; ++c)
-        __hip_atomic_store(&block_partials[(size_t)blockIdx.x * AGG + c], total.v[c], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the stores above have arrived before the ticket is drawn
-      s_is_last = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1 ? 1 : 0;
-    }
-    __syncthreads();
-    if (s_is_last) {
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-      Pack<V, AGG> share;
-      zero(share);
-      for (int j = tid; j < (int)gridDim.x; j += BLOCK) {
-#pragma unroll
-        for (int c = 0; c < AGG; ++c)
-          share.v[c] += __hip_atomic_load(&block_partials[(size_t)j * AGG + c], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      }
-      const Pack<V, AGG> all = block_total(share);
-      if (tid == 0) G::store_agg(p, all);
     }
   }
 }
@@ -1485,33 +1630,9 @@ fixup_kernel(const int* __restrict__ carry_row, const typename G::Value* __restr
 template <class G, int BLOCK>
 __global__ void __launch_bounds__(BLOCK)
 aggregate_kernel(const typename G::Params p, const typename G::Value* __restrict__ partials, const int count) {
-  using V = typename G::Value;
-  constexpr int AGG = G::AGG_WIDTH;
-  constexpr int NW = BLOCK / WAVE;
-  if constexpr (AGG > 0) {
-    __shared__ V s_wave_agg[NW][AGG];
-    Pack<V, AGG> acc;
-    zero(acc);
-    for (int j = threadIdx.x; j < count; j += BLOCK) {
-#pragma unroll
-      for (int c = 0; c < AGG; ++c) acc.v[c] += partials[(size_t)j * AGG + c];
-    }
-    wave_sum_to_last_lane<V, AGG>(acc.v);
-    if ((threadIdx.x & (WAVE - 1)) == WAVE - 1) {
-#pragma unroll
-      for (int c = 0; c < AGG; ++c) s_wave_agg[threadIdx.x / WAVE][c] = acc.v[c];
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      Pack<V, AGG> total;
-#pragma unroll
-      for (int c = 0; c < AGG; ++c) {
-        V s = s_wave_agg[0][c];
-        for (int w = 1; w < NW; ++w) s += s_wave_agg[w][c];
-        total.v[c] = s;
-      }
-      G::store_agg(p, total);
-    }
+  if constexpr (G::AGG_WIDTH > 0) {
+    const auto total = sum_partials<G, BLOCK, false>(partials, count);
+    if (threadIdx.x == 0) G::store_agg(p, total);
   }
 }
 

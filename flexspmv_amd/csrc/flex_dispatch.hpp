@@ -10,6 +10,7 @@
 #include <hip/hip_runtime.h>
 #include <hip/hip_ext.h>
 #include <stdint.h>
+#include <stddef.h>
 #include <stdio.h>
 #include <stdlib.h>
 
@@ -158,6 +159,19 @@ inline int resident_grid(KernelT kernel, int block_threads, GridCache& cache) {
 #define FLEX_TUNE_SINGLE_FIXUP_MAX_TILES 4096  // launches of at most this many tiles fold carries and aggregators in one block
 #endif
 constexpr int SINGLE_FIXUP_BLOCK = 1024;
+// A launch with counters (flexspmv_launch_args.counters) finishes itself, without a second kernel, up to 512 tiles of
+// 4-byte values or 256 of 8-byte values.  Such a launch runs for less than the 8 us it takes the host to issue two
+// kernels (2.7 to 4 us each): 256 x 256 Laplacian float32, 192 tiles, 8.2 -> 5.9 us a pass.  On the GPU the second kernel
+// is the cheaper way, by 0.5 us at 300 tiles and 1 us at 1 000 (blocks wait for their tickets, the records bypass the
+// caches), so larger launches, which the GPU's time decides, keep it (61 x 47 x 83 stencil: 9.4 against 8.4 us).
+constexpr int FINISH_MAX_TILES = FIXUP_BLOCK * FINISH_PER;
+template <typename V> constexpr int finish_max_tiles() { return FINISH_MAX_TILES * 4 / (int)sizeof(V); }
+static_assert((1 + FINISH_MAX_TILES / FINISH_GROUP) * 128 <= FLEXSPMV_COUNTER_BYTES, "a counter per group of blocks and one more");
+
+// args->counters, or none where the caller's struct ends before that field
+inline unsigned* counters_of(const flexspmv_launch_args* a) {
+  return a->struct_size >= sizeof(flexspmv_launch_args) ? (unsigned*)a->counters : nullptr;
+}
 
 template <class G, int BLOCK, int IPT, bool REDUCER>
 struct Dispatch {
@@ -170,7 +184,8 @@ struct Dispatch {
     int flat_blocks;
     bool search_in_blocks;
     bool single_fixup;
-    int fixup_per, fixup_blocks;  // tiles per thread of fixup_kernel, its blocks
+    bool can_finish;                          // the reducer's last block can do the fix-up
+    int fixup_block, fixup_per, fixup_blocks;  // threads of a fixup_kernel block, tiles per thread, blocks
     size_t off_coords, off_splits, off_carry_row, off_carry_val, off_partials, off_block_partials, off_ticket, total;
   };
 
@@ -249,9 +264,13 @@ struct Dispatch {
     l.off_carry_val = off;
     if (REDUCER) off += align_up(sizeof(V) * (size_t)l.num_tiles * (G::RED_WIDTH > 0 ? G::RED_WIDTH : 1));
     // (fixup_kernel: one block takes up to 8 tiles per thread; several blocks one, or eight where tiles hardly carry)
-    if (l.single_fixup) l.fixup_per = (l.num_tiles + SINGLE_FIXUP_BLOCK - 1) / SINGLE_FIXUP_BLOCK;
+    // A launch small enough to finish itself is folded by 256 threads either way: the same sums in the same order.
+    const bool small = l.single_fixup && l.num_tiles <= FINISH_MAX_TILES;
+    l.fixup_block = l.single_fixup && !small ? SINGLE_FIXUP_BLOCK : FIXUP_BLOCK;
+    if (l.single_fixup) l.fixup_per = (l.num_tiles + l.fixup_block - 1) / l.fixup_block;
     else l.fixup_per = l.tiling.snap_slack > 0 ? 8 : 1;
-    const int per_block = (l.single_fixup ? SINGLE_FIXUP_BLOCK : FIXUP_BLOCK) * l.fixup_per;
+    l.can_finish = small && l.num_tiles <= finish_max_tiles<V>() && BLOCK == FIXUP_BLOCK;
+    const int per_block = l.fixup_block * l.fixup_per;
     l.fixup_blocks = (l.num_tiles + per_block - 1) / per_block;
     l.off_partials = off;
     const size_t parts = REDUCER ? (size_t)l.num_tiles * partials_per_tile<BLOCK>() : (size_t)MAX_PERSISTENT_BLOCKS;
@@ -301,7 +320,7 @@ struct Dispatch {
     Layout l;
     const int bad = check(a, l, a->workspace == nullptr ? 0 : a->workspace_bytes);
     if (bad != FLEXSPMV_OK) return bad;
-    return launch(p, a, l, (char*)a->workspace);
+    return launch(p, a, l, (char*)a->workspace, counters_of(a));
   }
 
   // flexspmv_launch_static: the same launch with the library's own scratch; allocates nothing.
@@ -320,17 +339,18 @@ struct Dispatch {
     }
     char* ws = static_scratch();
     if (ws == nullptr) return FLEXSPMV_ERR_WORKSPACE;
-    return launch(p, a, l, ws);
+    return launch(p, a, l, ws, nullptr);
   }
   static constexpr size_t l_unbounded() { return ~(size_t)0; }
 
   // The kernels of one launch, on a->stream, with scratch at ws (l.total bytes, 256-byte aligned).
-  static int launch(const typename G::Params& p, const flexspmv_launch_args* a, const Layout& l, char* ws) {
+  static int launch(const typename G::Params& p, const flexspmv_launch_args* a, const Layout& l, char* ws, unsigned* counters) {
     static thread_local GridCache grid_cache;  // one per kernel instantiation and host thread
     hipStream_t stream = (hipStream_t)a->stream;
     const bool timed = (a->flags & FLEXSPMV_FLAG_TIME_KERNEL) != 0 && g_timer.ready();
     if (timed) g_timer.armed = false;  // untimed launches leave the last timed kernel's events readable
     const bool debug = (a->flags & FLEXSPMV_FLAG_DEBUG_SYNC) != 0 || debug_launch_env();
+    if (timed || debug) counters = nullptr;  // a launch that is timed or reported shows its kernels one by one
     int debug_rc = FLEXSPMV_OK;
     auto report = [&](const char* name, auto kernel, int grid, int block) {
       if (debug && debug_rc == FLEXSPMV_OK) debug_rc = debug_report(name, kernel, (unsigned)grid, (unsigned)block, stream);
@@ -384,46 +404,61 @@ struct Dispatch {
       constexpr int EPL = edges_per_load<G, IPT>();
       const bool wide_loads = EPL > 1 && l.tiling.snap_slack > 0 && nnz >= EPL;
       const Tiling& tl = l.tiling;
+#ifdef FLEX_TUNE_PERSISTENT
+      const bool finish = false;
+#else
+      const bool finish = counters != nullptr && l.can_finish;
+#endif
+      unsigned* marks = finish ? counters : ticket;
       auto launch_reducer = [&](auto kernel, const char* name) {
         if (timed) {
           hipExtLaunchKernelGGL(kernel, dim3(reduce_grid), dim3(BLOCK), 0, stream, g_timer.start, g_timer.stop, 0, coords,
                                 splits, row_end, source, tl.xcd_shift, tl.num_tiles, num_rows, nnz, tl.nominal,
-                                tl.snap_slack, tl.snap_mask, tl.row_group, p, carry_row, carry_val, partials, ticket);
+                                tl.snap_slack, tl.snap_mask, tl.row_group, p, carry_row, carry_val, partials, marks);
           g_timer.armed = true;
         } else {
           hipLaunchKernelGGL(kernel, dim3(reduce_grid), dim3(BLOCK), 0, stream, coords, splits, row_end, source,
                              tl.xcd_shift, tl.num_tiles, num_rows, nnz, tl.nominal, tl.snap_slack, tl.snap_mask,
-                             tl.row_group, p, carry_row, carry_val, partials, ticket);
+                             tl.row_group, p, carry_row, carry_val, partials, marks);
         }
         report(name, kernel, reduce_grid, BLOCK);
       };
-      if (wide_loads) launch_reducer(reduce_kernel<G, BLOCK, IPT, EPL>, "reduce_kernel (several edges per load)");
-      else launch_reducer(reduce_kernel<G, BLOCK, IPT, 1>, "reduce_kernel");
-      V* block_partials = (V*)(ws + l.off_block_partials);
-      constexpr int PARTS = partials_per_tile<BLOCK>();
-      auto launch_fixup = [&](auto kernel, const int block, const char* name) {
-        hipLaunchKernelGGL(kernel, dim3(l.fixup_blocks), dim3(block), 0, stream, (const int*)carry_row,
-                           (const V*)partials, (const V*)carry_val, l.num_tiles, l.fixup_per, block_partials, ticket, p);
-        report(name, kernel, l.fixup_blocks, block);
-      };
-      if (l.single_fixup) launch_fixup(fixup_kernel<G, SINGLE_FIXUP_BLOCK, PARTS>, SINGLE_FIXUP_BLOCK, "fixup_kernel (one block)");
-      else launch_fixup(fixup_kernel<G, FIXUP_BLOCK, PARTS>, FIXUP_BLOCK, "fixup_kernel");
+      if (finish) {
+        if (wide_loads) launch_reducer(reduce_kernel<G, BLOCK, IPT, EPL, true>, "reduce_kernel (several edges per load)");
+        else launch_reducer(reduce_kernel<G, BLOCK, IPT, 1, true>, "reduce_kernel");
+      } else {
+        if (wide_loads) launch_reducer(reduce_kernel<G, BLOCK, IPT, EPL, false>, "reduce_kernel (several edges per load)");
+        else launch_reducer(reduce_kernel<G, BLOCK, IPT, 1, false>, "reduce_kernel");
+        V* block_partials = (V*)(ws + l.off_block_partials);
+        constexpr int PARTS = partials_per_tile<BLOCK>();
+        auto launch_fixup = [&](auto kernel) {
+          hipLaunchKernelGGL(kernel, dim3(l.fixup_blocks), dim3(l.fixup_block), 0, stream, (const int*)carry_row,
+                             (const V*)partials, (const V*)carry_val, l.num_tiles, l.fixup_per, block_partials, ticket, p);
+          report(l.single_fixup ? "fixup_kernel (one block)" : "fixup_kernel", kernel, l.fixup_blocks, l.fixup_block);
+        };
+        if (l.fixup_block == SINGLE_FIXUP_BLOCK) launch_fixup(fixup_kernel<G, SINGLE_FIXUP_BLOCK, PARTS>);
+        else launch_fixup(fixup_kernel<G, FIXUP_BLOCK, PARTS>);
+      }
     } else {
-      int grid = resident_grid(flat_kernel<G, BLOCK, IPT>, BLOCK, grid_cache);
+      int grid = resident_grid(flat_kernel<G, BLOCK, IPT, false>, BLOCK, grid_cache);
       if (grid > l.num_tiles) grid = l.num_tiles;
       if (debug)
         fprintf(stderr, "[flexspmv] flat launch: %d edges, %d tiles of %d edges, %zu bytes of scratch\n", nnz, l.num_tiles,
                 TILE, l.total);
-      if (timed) {
-        hipExtLaunchKernelGGL((flat_kernel<G, BLOCK, IPT>), dim3(grid), dim3(BLOCK), 0, stream, g_timer.start,
-                              g_timer.stop, 0, p, nnz, l.num_tiles, partials);
-        g_timer.armed = true;
-      } else {
-        hipLaunchKernelGGL((flat_kernel<G, BLOCK, IPT>), dim3(grid), dim3(BLOCK), 0, stream, p, nnz, l.num_tiles,
-                           partials);
-      }
-      report("flat_kernel", flat_kernel<G, BLOCK, IPT>, grid, BLOCK);
-      if (G::AGG_WIDTH > 0) {
+      const bool finish = G::AGG_WIDTH > 0 && counters != nullptr && BLOCK == FIXUP_BLOCK && grid <= finish_max_tiles<V>();
+      auto launch_flat = [&](auto kernel) {
+        if (timed) {
+          hipExtLaunchKernelGGL(kernel, dim3(grid), dim3(BLOCK), 0, stream, g_timer.start, g_timer.stop, 0, p, nnz, l.num_tiles,
+                                partials, counters);
+          g_timer.armed = true;
+        } else {
+          hipLaunchKernelGGL(kernel, dim3(grid), dim3(BLOCK), 0, stream, p, nnz, l.num_tiles, partials, counters);
+        }
+        report("flat_kernel", kernel, grid, BLOCK);
+      };
+      if (finish) launch_flat(flat_kernel<G, BLOCK, IPT, (G::AGG_WIDTH > 0)>);
+      else launch_flat(flat_kernel<G, BLOCK, IPT, false>);
+      if (G::AGG_WIDTH > 0 && !finish) {
         hipLaunchKernelGGL((aggregate_kernel<G, FIXUP_BLOCK>), dim3(1), dim3(FIXUP_BLOCK), 0, stream, p,
                            (const V*)partials, grid);
         report("aggregate_kernel", aggregate_kernel<G, FIXUP_BLOCK>, 1, FIXUP_BLOCK);
@@ -437,7 +472,7 @@ struct Dispatch {
 
 inline int check_counts(const flexspmv_launch_args* a, int nv, int ni, int no) {
   if (a == nullptr) return fail(FLEXSPMV_ERR_BAD_ARGUMENT, "args is NULL");
-  if (a->struct_size != sizeof(flexspmv_launch_args))
+  if (a->struct_size != sizeof(flexspmv_launch_args) && a->struct_size != offsetof(flexspmv_launch_args, counters))
     return fail(FLEXSPMV_ERR_BAD_ARGUMENT, "struct_size does not match this library's flexspmv_launch_args");
   if ((a->flags & ~(FLEXSPMV_FLAG_TIME_KERNEL | FLEXSPMV_FLAG_REUSE_TILES | FLEXSPMV_FLAG_KEEP_TILES |
                     FLEXSPMV_FLAG_DEBUG_SYNC | FLEXSPMV_FLAG_SEARCH_TILES)) != 0)

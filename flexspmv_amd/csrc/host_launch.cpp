@@ -12,6 +12,7 @@
 
 #include <ATen/core/Tensor.h>
 #include <ATen/hip/EmptyTensor.h>
+#include <ATen/ops/zeros.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime_api.h>
@@ -20,7 +21,9 @@
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/utils/object_ptr.h>
 
+#include <map>
 #include <memory>
+#include <utility>
 #include <vector>
 
 #include "flexspmv.h"
@@ -114,6 +117,23 @@ PyObject* scratch_of(Launcher* self, PyObject* ext, const c10::Device& device, l
     return nullptr;
   }
   return made;
+}
+
+// Counters of launches on a stream of a device (flexspmv_launch_args.counters): cleared when they are made, left at zero
+// by every launch, shared by all libraries - launches on one stream are ordered.  Held under the GIL; made on the stream
+// they serve, so that the caching allocator hands a dropped block out again in that stream's order.  Never destroyed at
+// exit (the allocator may be gone by then).
+constexpr size_t MAX_COUNTERS = 64;
+void* counters_of(const c10::Device& device, hipStream_t stream) {
+  if (stream == hipStreamPerThread) return nullptr;  // one handle for a stream per thread
+  static auto* known = new std::map<std::pair<int, hipStream_t>, at::Tensor>();
+  const auto key = std::make_pair((int)device.index(), stream);
+  auto it = known->find(key);
+  if (it == known->end()) {
+    if (known->size() >= MAX_COUNTERS) known->clear();
+    it = known->emplace(key, at::zeros({FLEXSPMV_COUNTER_BYTES}, at::TensorOptions().dtype(at::kByte).device(device))).first;
+  }
+  return it->second.data_ptr();
 }
 
 constexpr int MAX_POINTERS = 64;  // of one kind; a library with more goes through Python
@@ -221,6 +241,7 @@ PyObject* launcher_launch(PyObject* self_obj, PyObject* const* call, Py_ssize_t 
   la.workspace = ws.data_ptr();
   la.workspace_bytes = (size_t)ws.numel();
   la.stream = stream;
+  la.counters = counters_of(device, stream);
   int rc;
   {
     pybind11::gil_scoped_release no_gil;

@@ -102,7 +102,13 @@ enum flexspmv_status {
  *                  they only have to be left alone between two launches when the second one carries
  *                  FLEXSPMV_FLAG_REUSE_TILES (and are worth leaving alone otherwise: see the tile table).
  *   stream         hipStream_t to launch on (NULL = default stream).  The call is asynchronous.
+ *   counters       NULL, or FLEXSPMV_COUNTER_BYTES of device memory, 128-byte aligned, that was zero when it was
+ *                  first given to a launch and that only launches of this package's libraries ordered with one
+ *                  another (one stream) have used since; every launch leaves it zero.  With it a launch of a few
+ *                  hundred tiles is one kernel (its last block folds what the others left) instead of two: the same
+ *                  results, bit for bit.  A struct_size that ends before this field means NULL.
  */
+#define FLEXSPMV_COUNTER_BYTES 8192
 typedef struct flexspmv_launch_args {
   uint32_t struct_size; /* sizeof(flexspmv_launch_args) */
   int32_t dtype;        /* enum flexspmv_dtype */
@@ -120,6 +126,7 @@ typedef struct flexspmv_launch_args {
   size_t workspace_bytes;
   void* stream;
   uint32_t flags; /* 0 or FLEXSPMV_FLAG_* */
+  void* counters;
 } flexspmv_launch_args;
 
 /* Run the fused sub-graph once.  Returns FLEXSPMV_OK, a negative flexspmv_status, or a hipError_t. */

@@ -1,0 +1,67 @@
+"""Small launches finish themselves (counters in the launch arguments): the same bits as with the fix-up in a kernel of
+its own, launch after launch, around the sizes where the route changes."""
+import pytest
+
+torch = pytest.importorskip("torch")
+
+from flexspmv_amd.binding import load_named
+
+pytestmark = pytest.mark.gpu
+
+# rows of the launches: one row, one tile, a few tiles, a group of 32 blocks and one more, both ends of the range of
+# 8-byte values (256 tiles), the end of the range of 4-byte values (512)
+ROWS = (1, 7, 240, 2_000, 12_000, 12_600, 98_000, 99_000, 196_000, 200_000)
+
+
+def rows_of(kind, n):
+    if kind == "even":
+        return torch.full((n,), 4, dtype=torch.int64)
+    length = torch.randint(0, 9, (n,), generator=torch.Generator().manual_seed(n))
+    length[n // 3] = min(9_000, 2 * n)           # carries through several tiles
+    length[-1] = max(int(length[-1]), 1)
+    return length
+
+
+@pytest.mark.parametrize("kind", ["even", "long row"])
+@pytest.mark.parametrize("n", ROWS)
+def test_reducer_launch_finishes_itself(n, kind):
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    length = rows_of(kind, n)
+    ptr = torch.zeros(n + 1, dtype=torch.int32)
+    ptr[1:] = torch.cumsum(length, 0)
+    ne = int(ptr[-1])
+    ptr = ptr.cuda()
+    col = torch.randint(0, n, (ne,), generator=gen, device="cuda", dtype=torch.int32)
+    rows = torch.repeat_interleave(torch.arange(n, dtype=torch.int32), length).cuda()
+    print(f"case one kernel {kind} {n} rows {ne} edges", flush=True)
+    for dtype in (torch.float32, torch.float64):
+        ext = load_named("spmv_dot", build_if_missing=False)
+        args = (torch.rand(ne, generator=gen, device="cuda", dtype=dtype),
+                torch.rand(n, generator=gen, device="cuda", dtype=dtype), col, rows, ptr, n, n)
+        want = ext._launch_checked(args, {})      # without counters: the fix-up is a kernel
+        for _ in range(4):                        # the counters are back at zero after every launch
+            got = ext.merged_spmv_launch(*args)
+            assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+    ext = load_named("index_spmv", build_if_missing=False)
+    w = torch.randint(-1000, 1000, (ne,), generator=gen, device="cuda")
+    ids = torch.randint(-1000, 1000, (n,), generator=gen, device="cuda")
+    each = w * ids[col.long()]
+    y, total = ext.merged_spmv_launch(w, ids, col, ptr, n, n)
+    assert torch.equal(y, torch.zeros(n, dtype=torch.int64, device="cuda").index_add_(0, rows.long(), each))
+    assert int(total) == int(each.sum())
+
+
+@pytest.mark.parametrize("n", [1, 2_047, 2_048, 2_049, 65_536, 524_288, 524_289, 1_048_576, 1_048_577, 3_000_000])
+def test_flat_launch_finishes_itself(n):
+    ext = load_named("mass_sum", build_if_missing=False)
+    dummy = torch.zeros(1, dtype=torch.int32, device="cuda")
+    print(f"case one kernel flat {n}", flush=True)
+    for dtype in (torch.float32, torch.float64):
+        h = torch.rand(n, device="cuda", dtype=dtype)
+        area = torch.rand(n, device="cuda", dtype=dtype)
+        (want,) = ext._launch_checked((h, area, dummy, n, n), {})
+        for _ in range(3):
+            (got,) = ext.merged_spmv_launch(h, area, dummy, n, n)
+            assert torch.equal(got, want)
+        exact = float((h.double() * area.double()).sum())
+        assert abs(float(got) - exact) <= 64 * torch.finfo(dtype).eps * exact
