@@ -170,13 +170,18 @@ class _DynamicCudaWrapper(nn.Module):
         self._output_shapes = list(output_shapes) if output_shapes is not None else None
         self._written_inputs = set(written_inputs)
         self._dummy_ro: Dict[torch.device, torch.Tensor] = {}
+        # positions of the call's arguments in the library's order, and which of them the kernel stores into
+        where = {n: i for i, n in enumerate(self._input_param_names)}
+        self._order = [where[n] for n in self._non_gather_value_inputs + self._gather_value_inputs]
+        self._cols_from = where[(self._gather_value_inputs or self._non_gather_value_inputs)[0]]
+        self._written_positions = [where[n] for n in self._input_param_names if n in self._written_inputs]
         # streamed edge tensors in the kernel's edge order, kept from the previous call: a tensor that has not
         # changed since (same storage, same version counter - a model parameter, a mesh constant) is not
         # permuted again
         self._sorted_inputs: Dict[str, Tuple] = {}
 
     def _on(self, name: str, device) -> torch.Tensor:
-        t = getattr(self, name)
+        t = self._buffers[name]
         if t.device != device:       # moved once, then kept: launches must see one unchanged tensor
             t = t.to(device)
             setattr(self, name, t)
@@ -199,48 +204,45 @@ class _DynamicCudaWrapper(nn.Module):
     def __call__(self, *args):
         if len(args) != len(self._input_param_names):
             raise RuntimeError(f"fused sub-module takes {len(self._input_param_names)} tensors, {len(args)} given")
-        for n, a in zip(self._input_param_names, args):
-            if n in self._written_inputs and not a.is_contiguous():
-                raise RuntimeError(f"{n} is written in place by the fused kernel and must be contiguous")
-        arg_map = {n: a.contiguous() for n, a in zip(self._input_param_names, args)}
-        device = next(iter(arg_map.values())).device
-
-        if self.row_end_offsets is not None:
-            ro = self._on("row_end_offsets", device)
-            num_rows = int(ro.numel() - 1)
+        for i in self._written_positions:
+            if not args[i].is_contiguous():
+                raise RuntimeError(f"{self._input_param_names[i]} is written in place by the fused kernel and must be "
+                                   f"contiguous")
+        device = args[0].device
+        ro = self._buffers["row_end_offsets"]
+        num_cols = args[self._cols_from].shape[0]
+        if ro is not None:
+            if ro.device != device:
+                ro = self._on("row_end_offsets", device)
+            num_rows = ro.shape[0] - 1
         else:
             ro = self._dummy_ro.get(device)
             if ro is None:          # no reducer: the binding still takes a tensor here
                 ro = torch.tensor([42], dtype=torch.int32, device=device)
                 self._dummy_ro[device] = ro
-            num_rows = None
-        gv = self._gather_value_inputs[0] if self._gather_value_inputs else self._non_gather_value_inputs[0]
-        num_cols = int(arg_map[gv].shape[0])
-        if num_rows is None:
             num_rows = num_cols
 
-        perm = None
-        if self.edge_permutation is not None:
+        call_args = [args[i] if args[i].is_contiguous() else args[i].contiguous() for i in self._order]
+        perm = self._buffers["edge_permutation"]
+        if perm is not None:
             perm = self._on("edge_permutation", device)
             if perm.is_cuda and perm.dtype != torch.int32:      # the permutation kernels take int32
                 perm = perm.to(torch.int32)
                 self.edge_permutation = perm
-            for n in self._non_gather_value_inputs:
-                arg_map[n] = self._in_edge_order(n, arg_map[n], perm)
-        call_args = [arg_map[n] for n in self._non_gather_value_inputs]
-        call_args += [arg_map[n] for n in self._gather_value_inputs]
+            for k, n in enumerate(self._non_gather_value_inputs):
+                call_args[k] = self._in_edge_order(n, call_args[k], perm)
         call_args += [self._on(b, device) for b in self._selector_buf_names]
-        call_args += [ro, num_rows, num_cols]
 
-        outs = self._ext.merged_spmv_launch(*call_args)
+        outs = self._ext.merged_spmv_launch(*call_args, ro, num_rows, num_cols)
         # The kernel stored into the written inputs through raw pointers: their version counters go up as they
         # would after torch's own in-place operations, so that nobody (this class's copies of unchanged edge
         # tensors in another wrapper included) mistakes them for unchanged.
-        for n, a in zip(self._input_param_names, args):
-            if n in self._written_inputs:
-                if perm is not None and n in self._non_gather_value_inputs:
-                    scatter_edges(arg_map[n], perm, out=a)      # stores went to the sorted copy: put them back
-                _mark_written(a)
+        for i in self._written_positions:
+            if perm is not None:
+                n = self._input_param_names[i]
+                if n in self._non_gather_value_inputs:      # stores went to the sorted copy: put them back
+                    scatter_edges(call_args[self._non_gather_value_inputs.index(n)], perm, out=args[i])
+            _mark_written(args[i])
         if outs is None:
             return []
         outs = list(outs) if isinstance(outs, (tuple, list)) else [outs]
@@ -248,7 +250,8 @@ class _DynamicCudaWrapper(nn.Module):
             outs = [scatter_edges(o, perm) if per_edge else o
                     for o, per_edge in zip(outs, self._per_edge_outputs)]
         if self._output_shapes is not None and len(self._output_shapes) == len(outs):
-            outs = [o.view(s) if s and o.numel() == _numel(s) else o for o, s in zip(outs, self._output_shapes)]
+            outs = [o if not s or o.shape == s or o.numel() != _numel(s) else o.view(s)
+                    for o, s in zip(outs, self._output_shapes)]
         return outs
 
 
