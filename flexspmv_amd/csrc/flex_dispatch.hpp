@@ -168,6 +168,13 @@ constexpr int FINISH_MAX_TILES = FIXUP_BLOCK * FINISH_PER;
 template <typename V> constexpr int finish_max_tiles() { return FINISH_MAX_TILES * 4 / (int)sizeof(V); }
 static_assert((1 + FINISH_MAX_TILES / FINISH_GROUP) * 128 <= FLEXSPMV_COUNTER_BYTES, "a counter per group of blocks and one more");
 
+// A flat launch of few edges gives every thread 1, 2 or 4 of them instead of IPT, as long as that makes at most a block
+// per CU: with tiles of 2 048 edges 45 000 edges keep 22 of the 256 CUs busy.  Per pass, IPT = 8 against this rule:
+// map_store float64 45 000 edges 7.0 -> 4.9 us, 135 000 7.25 -> 6.2, 200 000 7.9 -> 7.0; mass_sum, which reads two words
+// an edge and waits for its launch, 4.6 -> 4.4 at 100 000.  More blocks than CUs are slower (135 000 edges, two and four
+// blocks a CU: 7.5, 7.6 us), and so is anything but IPT edges a thread once there is a block of them per CU.
+constexpr int FLAT_SMALL_BLOCKS = NUM_CUS;
+
 // args->counters, or none where the caller's struct ends before that field
 inline unsigned* counters_of(const flexspmv_launch_args* a) {
   return a->struct_size >= sizeof(flexspmv_launch_args) ? (unsigned*)a->counters : nullptr;
@@ -440,29 +447,42 @@ struct Dispatch {
         else launch_fixup(fixup_kernel<G, FIXUP_BLOCK, PARTS>);
       }
     } else {
-      int grid = resident_grid(flat_kernel<G, BLOCK, IPT, false>, BLOCK, grid_cache);
-      if (grid > l.num_tiles) grid = l.num_tiles;
-      if (debug)
-        fprintf(stderr, "[flexspmv] flat launch: %d edges, %d tiles of %d edges, %zu bytes of scratch\n", nnz, l.num_tiles,
-                TILE, l.total);
-      const bool finish = G::AGG_WIDTH > 0 && counters != nullptr && BLOCK == FIXUP_BLOCK && grid <= finish_max_tiles<V>();
-      auto launch_flat = [&](auto kernel) {
-        if (timed) {
-          hipExtLaunchKernelGGL(kernel, dim3(grid), dim3(BLOCK), 0, stream, g_timer.start, g_timer.stop, 0, p, nnz, l.num_tiles,
-                                partials, counters);
-          g_timer.armed = true;
-        } else {
-          hipLaunchKernelGGL(kernel, dim3(grid), dim3(BLOCK), 0, stream, p, nnz, l.num_tiles, partials, counters);
+      // edges per thread: as few as make at most FLAT_SMALL_BLOCKS blocks, at most IPT
+      auto launch_with = [&](auto ipt_tag) {
+        constexpr int ITEMS = decltype(ipt_tag)::value, FLAT_TILE = BLOCK * ITEMS;
+        const int num_tiles = (int)((a->ne + FLAT_TILE - 1) / FLAT_TILE);
+        int grid = num_tiles;
+        if (ITEMS == IPT) {  // a launch of any size: no more blocks than are resident at once, each walks its tiles
+          grid = resident_grid(flat_kernel<G, BLOCK, IPT, false>, BLOCK, grid_cache);
+          if (grid > num_tiles) grid = num_tiles;
         }
-        report("flat_kernel", kernel, grid, BLOCK);
+        if (debug)
+          fprintf(stderr, "[flexspmv] flat launch: %d edges, %d tiles of %d edges, %zu bytes of scratch\n", nnz, num_tiles,
+                  FLAT_TILE, l.total);
+        const bool finish = G::AGG_WIDTH > 0 && counters != nullptr && BLOCK == FIXUP_BLOCK && grid <= finish_max_tiles<V>();
+        auto launch_flat = [&](auto kernel) {
+          if (timed) {
+            hipExtLaunchKernelGGL(kernel, dim3(grid), dim3(BLOCK), 0, stream, g_timer.start, g_timer.stop, 0, p, nnz, num_tiles,
+                                  partials, counters);
+            g_timer.armed = true;
+          } else {
+            hipLaunchKernelGGL(kernel, dim3(grid), dim3(BLOCK), 0, stream, p, nnz, num_tiles, partials, counters);
+          }
+          report("flat_kernel", kernel, grid, BLOCK);
+        };
+        if (finish) launch_flat(flat_kernel<G, BLOCK, ITEMS, (G::AGG_WIDTH > 0)>);
+        else launch_flat(flat_kernel<G, BLOCK, ITEMS, false>);
+        if (G::AGG_WIDTH > 0 && !finish) {
+          hipLaunchKernelGGL((aggregate_kernel<G, FIXUP_BLOCK>), dim3(1), dim3(FIXUP_BLOCK), 0, stream, p,
+                             (const V*)partials, grid);
+          report("aggregate_kernel", aggregate_kernel<G, FIXUP_BLOCK>, 1, FIXUP_BLOCK);
+        }
       };
-      if (finish) launch_flat(flat_kernel<G, BLOCK, IPT, (G::AGG_WIDTH > 0)>);
-      else launch_flat(flat_kernel<G, BLOCK, IPT, false>);
-      if (G::AGG_WIDTH > 0 && !finish) {
-        hipLaunchKernelGGL((aggregate_kernel<G, FIXUP_BLOCK>), dim3(1), dim3(FIXUP_BLOCK), 0, stream, p,
-                           (const V*)partials, grid);
-        report("aggregate_kernel", aggregate_kernel<G, FIXUP_BLOCK>, 1, FIXUP_BLOCK);
-      }
+      const int64_t threads = (int64_t)BLOCK * FLAT_SMALL_BLOCKS;
+      if (IPT > 1 && a->ne <= threads) launch_with(std::integral_constant<int, 1>{});
+      else if (IPT > 2 && a->ne <= 2 * threads) launch_with(std::integral_constant<int, (IPT > 2 ? 2 : IPT)>{});
+      else if (IPT > 4 && a->ne <= 4 * threads) launch_with(std::integral_constant<int, (IPT > 4 ? 4 : IPT)>{});
+      else launch_with(std::integral_constant<int, IPT>{});
     }
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail_hip(e, "kernel launch failed");

@@ -65,3 +65,23 @@ def test_flat_launch_finishes_itself(n):
             assert torch.equal(got, want)
         exact = float((h.double() * area.double()).sum())
         assert abs(float(got) - exact) <= 64 * torch.finfo(dtype).eps * exact
+
+
+# edges per thread of a flat launch: 1 up to 256 blocks of 256 edges, then 2, 4 and 8; one edge to each side of every change
+@pytest.mark.parametrize("n", [1, 255, 257, 65_535, 65_536, 65_537, 131_072, 131_073, 262_144, 262_145])
+def test_flat_launch_edges_per_thread(n):
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    dummy = torch.zeros(1, dtype=torch.int32, device="cuda")
+    v = n // 3 + 1
+    near = torch.randint(0, v, (n,), generator=gen, device="cuda", dtype=torch.int32)
+    print(f"case edges per thread {n}", flush=True)
+    for dtype in (torch.float32, torch.float64):
+        eps = torch.finfo(dtype).eps
+        a = torch.rand((n, 3), generator=gen, device="cuda", dtype=dtype)
+        b = torch.rand((v, 3), generator=gen, device="cuda", dtype=dtype)
+        ext = load_named("map_store", build_if_missing=False)
+        store, total = ext.merged_spmv_launch(a, b, near, dummy, v, v)
+        exact = a.double() * b.double()[near.long()]
+        assert bool(((store.double() - (exact + 1.0)).abs() <= 2 * eps * (exact + 1.0)).all())   # a product and a sum
+        # a thread adds up to 8 edges, a wavefront 64 threads, a block 4 wavefronts, the last block 256: 24 links
+        assert bool(((total.double() - exact.sum(0)).abs() <= 32 * eps * exact.sum(0)).all())
