@@ -164,10 +164,14 @@ constexpr int SINGLE_FIXUP_BLOCK = 1024;
 // kernels (2.7 to 4 us each): 256 x 256 Laplacian float32, 192 tiles, 8.2 -> 5.9 us a pass.  On the GPU the second kernel
 // is the cheaper way, by 0.5 us at 300 tiles and 1 us at 1 000 (blocks wait for their tickets, the records bypass the
 // caches), so larger launches, which the GPU's time decides, keep it (61 x 47 x 83 stencil: 9.4 against 8.4 us).
-constexpr int FINISH_MAX_TILES = FIXUP_BLOCK * FINISH_PER;
+// Where there is no aggregator and tiles start on rows, blocks arrive early and the last one rarely has anything to fold:
+// such launches finish themselves up to 1 024 tiles.
+// (512 x 512 points, 1 024 tiles: float32 8.2 -> 7.3 us, float64 9.3 -> 8.4 against two kernels; with the 8 tiles a thread that
+// 2 000 tiles would need, the kernel's registers cost it a block per CU.)
+constexpr int FINISH_MAX_TILES = FIXUP_BLOCK * 2;
+constexpr int FINISH_EARLY_MAX_TILES = FIXUP_BLOCK * 4;
 template <typename V> constexpr int finish_max_tiles() { return FINISH_MAX_TILES * 4 / (int)sizeof(V); }
-static_assert((1 + FINISH_MAX_TILES / FINISH_GROUP) * 128 <= FLEXSPMV_COUNTER_BYTES, "a counter per group of blocks and one more");
-
+static_assert((1 + FINISH_EARLY_MAX_TILES / FINISH_GROUP) * 128 <= FLEXSPMV_COUNTER_BYTES, "a counter per group of blocks and one more");
 // A flat launch of few edges gives every thread 1, 2 or 4 of them instead of IPT, as long as that makes at most a block
 // per CU: with tiles of 2 048 edges 45 000 edges keep 22 of the 256 CUs busy.  Per pass, IPT = 8 against this rule:
 // map_store float64 45 000 edges 7.0 -> 4.9 us, 135 000 7.25 -> 6.2, 200 000 7.9 -> 7.0; mass_sum, which reads two words
@@ -198,7 +202,9 @@ struct Dispatch {
 
   // Row-snapped tiles pay with smaller tiles (capacity minus the slack a boundary may be moved by), so
   // they are used where a line's worth of rows is a small part of a tile: the slack is the merge items
-  // of that many average rows, and snapping is off when it exceeds an eighth of the tile.
+  // of that many rows of the average length, rounded up (a stencil's interior rows are a little longer than its average
+  // one: with the plain average 1 boundary in 50 of a 3-D stencil stayed where it was and left a carry to fold), and
+  // snapping is off when it exceeds an eighth of the tile.
   static Tiling tiling_for(int64_t num_rows, int64_t ne) {
     Tiling t;
     t.nominal = TILE;
@@ -208,7 +214,7 @@ struct Dispatch {
     t.row_group = 0;
     if (REDUCER && FLEX_TUNE_SNAP_BYTES > 0 && num_rows > 0) {
       const int snap_rows = FLEX_TUNE_SNAP_BYTES / (int)sizeof(V) > 1 ? FLEX_TUNE_SNAP_BYTES / (int)sizeof(V) : 1;
-      const int64_t slack = (snap_rows * (num_rows + ne) + num_rows - 1) / num_rows;  // snap_rows average rows
+      const int64_t slack = snap_rows * ((num_rows + ne + num_rows - 1) / num_rows);
       if (slack <= TILE / 8) {
         t.snap_slack = (int)slack;
         t.snap_mask = snap_rows - 1;
@@ -272,11 +278,12 @@ struct Dispatch {
     if (REDUCER) off += align_up(sizeof(V) * (size_t)l.num_tiles * (G::RED_WIDTH > 0 ? G::RED_WIDTH : 1));
     // (fixup_kernel: one block takes up to 8 tiles per thread; several blocks one, or eight where tiles hardly carry)
     // A launch small enough to finish itself is folded by 256 threads either way: the same sums in the same order.
-    const bool small = l.single_fixup && l.num_tiles <= FINISH_MAX_TILES;
+    const bool early = G::AGG_WIDTH == 0 && l.tiling.snap_slack > 0;
+    const bool small = l.single_fixup && l.num_tiles <= (early ? FINISH_EARLY_MAX_TILES : FINISH_MAX_TILES);
     l.fixup_block = l.single_fixup && !small ? SINGLE_FIXUP_BLOCK : FIXUP_BLOCK;
     if (l.single_fixup) l.fixup_per = (l.num_tiles + l.fixup_block - 1) / l.fixup_block;
     else l.fixup_per = l.tiling.snap_slack > 0 ? 8 : 1;
-    l.can_finish = small && l.num_tiles <= finish_max_tiles<V>() && BLOCK == FIXUP_BLOCK;
+    l.can_finish = small && (early || l.num_tiles <= finish_max_tiles<V>()) && BLOCK == FIXUP_BLOCK;
     const int per_block = l.fixup_block * l.fixup_per;
     l.fixup_blocks = (l.num_tiles + per_block - 1) / per_block;
     l.off_partials = off;
@@ -431,11 +438,13 @@ struct Dispatch {
         report(name, kernel, reduce_grid, BLOCK);
       };
       if (finish) {
-        if (wide_loads) launch_reducer(reduce_kernel<G, BLOCK, IPT, EPL, true>, "reduce_kernel (several edges per load)");
-        else launch_reducer(reduce_kernel<G, BLOCK, IPT, 1, true>, "reduce_kernel");
+        constexpr bool CAN_EARLY = G::AGG_WIDTH == 0;
+        if (wide_loads) launch_reducer(reduce_kernel<G, BLOCK, IPT, EPL, true, CAN_EARLY>, "reduce_kernel (several edges per load)");
+        else if (CAN_EARLY && tl.snap_slack > 0) launch_reducer(reduce_kernel<G, BLOCK, IPT, 1, true, CAN_EARLY>, "reduce_kernel");
+        else launch_reducer(reduce_kernel<G, BLOCK, IPT, 1, true, false>, "reduce_kernel");
       } else {
-        if (wide_loads) launch_reducer(reduce_kernel<G, BLOCK, IPT, EPL, false>, "reduce_kernel (several edges per load)");
-        else launch_reducer(reduce_kernel<G, BLOCK, IPT, 1, false>, "reduce_kernel");
+        if (wide_loads) launch_reducer(reduce_kernel<G, BLOCK, IPT, EPL, false, false>, "reduce_kernel (several edges per load)");
+        else launch_reducer(reduce_kernel<G, BLOCK, IPT, 1, false, false>, "reduce_kernel");
         V* block_partials = (V*)(ws + l.off_block_partials);
         constexpr int PARTS = partials_per_tile<BLOCK>();
         auto launch_fixup = [&](auto kernel) {

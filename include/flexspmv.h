@@ -172,7 +172,8 @@ int flexspmv_last_kernel_ms(float* ms);
  *                        nominal + snap_slack, and more where a cap on the rows per tile shortens nominal
  *   out[5] search_in_blocks  1 when a launch with FLEXSPMV_FLAG_SEARCH_TILES searches inside the reducer blocks,
  *                        0 when it runs a search kernel (launches without the flag never run one)
- * For libraries without a reducer the tiles are plain edge ranges of `nominal` edges.
+ * For libraries without a reducer the tiles are plain edge ranges of `nominal` edges (launches of so few edges
+ * that there is less than such a tile per CU cut them further).
  * Returns FLEXSPMV_OK, FLEXSPMV_ERR_BAD_DTYPE or FLEXSPMV_ERR_TOO_LARGE. */
 int flexspmv_tiling(int32_t dtype, int64_t num_rows, int64_t ne, int32_t out[6]);
 

@@ -85,3 +85,30 @@ def test_flat_launch_edges_per_thread(n):
         assert bool(((store.double() - (exact + 1.0)).abs() <= 2 * eps * (exact + 1.0)).all())   # a product and a sum
         # a thread adds up to 8 edges, a wavefront 64 threads, a block 4 wavefronts, the last block 256: 24 links
         assert bool(((total.double() - exact.sum(0)).abs() <= 32 * eps * exact.sum(0)).all())
+
+
+# Without an aggregator, blocks whose tile has no carry arrive early: one row to two tiles, a group of 32 blocks and one
+# more, and the end of the range (1 024 tiles of 256 rows) to both sides.  "long row": some tiles carry, most do not.
+@pytest.mark.parametrize("kind", ["even", "long row"])
+@pytest.mark.parametrize("n", (1, 255, 257, 8_192, 8_193, 65_000, 262_144, 262_400))
+def test_blocks_arrive_early(n, kind):
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    length = rows_of(kind, n)
+    other = length.flip(0).contiguous()          # another matrix behind the same row pointer: the tile table is refused
+    print(f"case early {kind} {n} rows", flush=True)
+    ext = load_named("csr_spmv", build_if_missing=False)
+    ptr = torch.zeros(n + 1, dtype=torch.int32, device="cuda")
+    for dtype in (torch.float32, torch.float64):
+        for lengths in (length, other, length):
+            ptr[1:] = torch.cumsum(lengths, 0).cuda()
+            ne = int(ptr[-1])
+            col = torch.randint(0, n, (ne,), generator=gen, device="cuda", dtype=torch.int32)
+            rows = torch.repeat_interleave(torch.arange(n), lengths).cuda()
+            a = torch.rand(ne, generator=gen, device="cuda", dtype=dtype)
+            x = torch.rand(n, generator=gen, device="cuda", dtype=dtype)
+            got = [ext.merged_spmv_launch(a, x, col, ptr, n, n)[0] for _ in range(3)]
+            (want,) = ext._launch_checked((a, x, col, ptr, n, n), {})      # without counters: the fix-up is a kernel
+            assert all(torch.equal(y, want) for y in got)
+            exact = torch.zeros(n, dtype=torch.float64, device="cuda").index_add_(0, rows, a.double() * x.double()[col.long()])
+            # every term positive: at most a rounding per term of the longest row
+            assert bool(((want.double() - exact).abs() <= int(lengths.max()) * torch.finfo(dtype).eps * exact).all())
