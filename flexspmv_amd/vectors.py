@@ -9,7 +9,7 @@ from typing import Optional, Tuple
 
 from . import build as _build
 
-ABI_VERSION = 1
+ABI_VERSION = 2
 MAX_PARTIALS = 2048          # FLEXSPMV_CG_MAX_PARTIALS
 EXPORTED_SYMBOLS = ("flexspmv_cg_step", "flexspmv_cg_direction", "flexspmv_vectors_last_error",
                     "flexspmv_vectors_abi_version")
@@ -25,9 +25,9 @@ def load_library(path: Optional[str] = None) -> ctypes.CDLL:
     import torch  # noqa: F401  (torch's HIP runtime has to be the one in the process)
     lib = ctypes.CDLL(path, mode=ctypes.RTLD_LOCAL)
     vp, i64, i32 = ctypes.c_void_p, ctypes.c_int64, ctypes.c_int
-    lib.flexspmv_cg_step.argtypes = [vp, vp, vp, vp, vp, vp, i64, i32, vp, vp]
+    lib.flexspmv_cg_step.argtypes = [vp, vp, vp, vp, i64, i32, vp, vp]
     lib.flexspmv_cg_step.restype = ctypes.c_int
-    lib.flexspmv_cg_direction.argtypes = [vp, vp, vp, vp, vp, vp, i64, i32, vp]
+    lib.flexspmv_cg_direction.argtypes = [vp, vp, vp, vp, vp, vp, vp, vp, i64, i32, vp]
     lib.flexspmv_cg_direction.restype = ctypes.c_int
     lib.flexspmv_vectors_last_error.argtypes = []
     lib.flexspmv_vectors_last_error.restype = ctypes.c_char_p
@@ -75,11 +75,12 @@ class ConjugateGradientUpdates:
         rr_new = torch.empty_like(rr)
         with torch.cuda.device(self._device):
             stream = torch.cuda.current_stream().cuda_stream
-            rc = lib.flexspmv_cg_step(x.data_ptr(), r.data_ptr(), p.data_ptr(), ap.data_ptr(), rr.data_ptr(),
-                                      pap.data_ptr(), n, self._bytes, self._partials.data_ptr(), stream)
+            rc = lib.flexspmv_cg_step(r.data_ptr(), ap.data_ptr(), rr.data_ptr(), pap.data_ptr(), n, self._bytes,
+                                      self._partials.data_ptr(), stream)
             if rc == 0:
-                rc = lib.flexspmv_cg_direction(p_next.data_ptr(), p.data_ptr(), r.data_ptr(), rr.data_ptr(),
-                                               rr_new.data_ptr(), self._partials.data_ptr(), n, self._bytes, stream)
+                rc = lib.flexspmv_cg_direction(x.data_ptr(), p_next.data_ptr(), p.data_ptr(), r.data_ptr(), rr.data_ptr(),
+                                               pap.data_ptr(), rr_new.data_ptr(), self._partials.data_ptr(), n,
+                                               self._bytes, stream)
         if rc != 0:
             raise RuntimeError(f"flexspmv vector update failed ({rc}): {lib.flexspmv_vectors_last_error().decode()}")
         return p_next, rr_new

@@ -18,7 +18,7 @@
 extern "C" {
 #endif
 
-#define FLEXSPMV_VECTORS_ABI_VERSION 1
+#define FLEXSPMV_VECTORS_ABI_VERSION 2
 
 /* Return codes (negative); positive values are hipError_t codes passed through unchanged. */
 enum flexspmv_vectors_status {
@@ -29,16 +29,16 @@ enum flexspmv_vectors_status {
 /* Values the partials of flexspmv_cg_step take (value_bytes each), whatever n is. */
 #define FLEXSPMV_CG_MAX_PARTIALS 2048
 
-/* x += alpha p and r -= alpha ap with alpha = rr / pap (both one value), and what the blocks add to the new r . r.
- * value_bytes: 4 (float) or 8 (double).  x, r: updated in place; p, ap: read; partials: FLEXSPMV_CG_MAX_PARTIALS
- * values, filled as far as flexspmv_cg_direction with the same n reads them.  No array may overlap another. */
-int flexspmv_cg_step(void* x, void* r, const void* p, const void* ap, const void* rr, const void* pap, int64_t n,
-                     int value_bytes, void* partials, void* stream);
+/* r -= alpha ap with alpha = rr / pap (both one value), and what the blocks add to the new r . r.
+ * value_bytes: 4 (float) or 8 (double).  r: updated in place; ap: read; partials: FLEXSPMV_CG_MAX_PARTIALS values,
+ * filled as far as flexspmv_cg_direction with the same n reads them.  No array may overlap another. */
+int flexspmv_cg_step(void* r, const void* ap, const void* rr, const void* pap, int64_t n, int value_bytes, void* partials,
+                     void* stream);
 
-/* rr_new = sum of the partials (in a fixed order) and p_next = r + (rr_new / rr) p.  p_next may be p; rr_new must
- * not be rr. */
-int flexspmv_cg_direction(void* p_next, const void* p, const void* r, const void* rr, void* rr_new,
-                          const void* partials, int64_t n, int value_bytes, void* stream);
+/* x += alpha p with the same alpha (x: updated in place), rr_new = sum of the partials (in a fixed order) and
+ * p_next = r + (rr_new / rr) p.  p_next may be p; rr_new must not be rr or pap; no other arrays may overlap. */
+int flexspmv_cg_direction(void* x, void* p_next, const void* p, const void* r, const void* rr, const void* pap,
+                          void* rr_new, const void* partials, int64_t n, int value_bytes, void* stream);
 
 /* Message of the last failed call on this thread ("" if none). */
 const char* flexspmv_vectors_last_error(void);
