@@ -1094,17 +1094,21 @@ reduce_tile(const int tile, const int2 c0, const int2 c1, const Tiling& tl, cons
 //       continue an earlier run and leave them alone.
 // The same sums in the same order on every run, no floating-point atomics.
 //
-// Launches of at most 512 tiles (1 024 where blocks arrive early) are folded by 256 threads (the reducer's last block, or a kernel of one block), those of
-// a few thousand by one block of 1024.  Larger ones use blocks of 256 threads: a tile per thread where tiles carry, eight
-// on row-snapped launches.  With several blocks the one that draws the last ticket adds the blocks' aggregator sums, in
-// block order.  What it reads was stored write-through at device scope and had arrived before the ticket was drawn, so no
-// block has to write its XCD's L2 back: that release cost 15 us a launch, a kernel of its own for the sum 4.7.
-// Whole passes, against loads one tile after the other and the sum in a kernel of its own: spring-mass 100^3 25.9 ->
-// 25.0 us, rows of 18 to 81 entries (301 000 of them, float64) 43.5 -> 42.7, Poisson 256^3 308.6 -> 308.3.
+// Small launches (flex_dispatch.hpp says which) are folded by 256 threads: the reducer's last block, or a kernel of one
+// block.  Larger ones use blocks of 256 threads with a tile per thread: where tiles carry, one block with several tiles a
+// thread spends longer on its runs than blocks side by side.
+// Aggregators up to 8 192 tiles: one more block, which only adds up the partials, beside blocks of 1 024 threads that
+// only fold carries, so that none waits for another.  Beyond, the block that draws the last ticket adds the blocks' sums,
+// in block order.  What it reads was stored write-through at device scope and had arrived before the ticket was drawn, so
+// no block has to write its XCD's L2 back: that release cost 15 us a launch, a kernel of its own for the sum 4.7.
+// Per pass, one block of 1 024 threads up to 4 096 tiles (8 192 row-snapped ones) -> this: 200 000 rows of 20 to 50
+// entries, float32 31.2 -> 18.0 us; R-MAT scale 19 float32 44.4 -> 34.1, float64 63.6 -> 50.7, int64 sums 67.1 -> 53.9;
+// spring-mass 100^3 24.3 -> 23.3.
 // ----------------------------------------------------------------------------------------------
 
 // Tiles [first, first + BLOCK * PER).  acc: receives the thread's share of the aggregators.
-template <class G, int BLOCK, int PARTS_PER_TILE, int PER, bool FINISH>
+// SUMS: (false) another block adds up the partials.
+template <class G, int BLOCK, int PARTS_PER_TILE, int PER, bool FINISH, bool SUMS>
 __device__ __forceinline__ void
 fold_tiles(const typename G::Params& p, const int first, const int num_tiles, const int* __restrict__ carry_row,
            const typename G::Value* __restrict__ carry_val, const typename G::Value* __restrict__ agg_partials,
@@ -1113,7 +1117,7 @@ fold_tiles(const typename G::Params& p, const int first, const int num_tiles, co
   constexpr int RED = G::RED_WIDTH, AGG = G::AGG_WIDTH;
   constexpr int REDN = RED > 0 ? RED : 1;
   constexpr int NW = BLOCK / WAVE;
-  constexpr int PARTS = AGG > 0 ? PARTS_PER_TILE * AGG : 1;
+  constexpr int PARTS = AGG > 0 && SUMS ? PARTS_PER_TILE * AGG : 0;
   __shared__ int s_vote[NW];
   __shared__ int s_key[NW];
   __shared__ V s_val[NW][REDN];
@@ -1129,7 +1133,7 @@ fold_tiles(const typename G::Params& p, const int first, const int num_tiles, co
   {
     // neighbouring lanes take neighbouring tiles here: everything in whole lines
     int row[PER], before[PER], after[PER];
-    V part[PER][PARTS];
+    V part[PER][PARTS > 0 ? PARTS : 1];
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
       const int t = min(first + i * BLOCK + tid, last);
@@ -1137,7 +1141,7 @@ fold_tiles(const typename G::Params& p, const int first, const int num_tiles, co
       before[i] = get_word<FINISH>(carry_row + max(t - 1, 0));
       after[i] = get_word<FINISH>(carry_row + min(t + 1, last));
 #pragma unroll
-      for (int c = 0; c < (AGG > 0 ? PARTS : 0); ++c) part[i][c] = get_word<FINISH>(agg_partials + ((size_t)t * PARTS + c));
+      for (int c = 0; c < PARTS; ++c) part[i][c] = get_word<FINISH>(agg_partials + ((size_t)t * PARTS + c));
     }
     bool any = false, runs = false;
 #pragma unroll
@@ -1148,7 +1152,7 @@ fold_tiles(const typename G::Params& p, const int first, const int num_tiles, co
       any |= row[i] >= 0;
       runs |= row[i] >= 0 && ((t > 0 && before[i] == row[i]) || (t < last && after[i] == row[i]));
 #pragma unroll
-      for (int c = 0; c < (AGG > 0 ? PARTS : 0); ++c) acc.v[c % (AGG > 0 ? AGG : 1)] += t <= last ? part[i][c] : V(0);
+      for (int c = 0; c < PARTS; ++c) acc.v[c % (AGG > 0 ? AGG : 1)] += t <= last ? part[i][c] : V(0);
     }
     if constexpr (RED > 0) {
       const int mine = (__builtin_amdgcn_ballot_w64(any) != 0ull ? 1 : 0) | (__builtin_amdgcn_ballot_w64(runs) != 0ull ? 2 : 0);
@@ -1343,18 +1347,18 @@ fold_tiles(const typename G::Params& p, const int first, const int num_tiles, co
   }
 }
 
-// ... `per` tiles per thread, uniform over the launch, at most MAX_PER (2 or 8) of them
-template <class G, int BLOCK, int PARTS_PER_TILE, int MAX_PER, bool FINISH>
+// ... `per` tiles per thread, uniform over the launch, at most MAX_PER of them
+template <class G, int BLOCK, int PARTS_PER_TILE, int MAX_PER, bool FINISH, bool SUMS>
 __device__ __forceinline__ void
 fixup_tiles(const typename G::Params& p, const int block, const int num_tiles, const int per,
             const int* __restrict__ carry_row, const typename G::Value* __restrict__ carry_val,
             const typename G::Value* __restrict__ agg_partials, Pack<typename G::Value, G::AGG_WIDTH>& acc) {
   auto fold = [&](auto per_tag) {
     constexpr int PER = decltype(per_tag)::value;
-    fold_tiles<G, BLOCK, PARTS_PER_TILE, PER, FINISH>(p, block * BLOCK * PER, num_tiles, carry_row, carry_val, agg_partials, acc);
+    fold_tiles<G, BLOCK, PARTS_PER_TILE, PER, FINISH, SUMS>(p, block * BLOCK * PER, num_tiles, carry_row, carry_val, agg_partials, acc);
   };
-  if (per == 1) fold(std::integral_constant<int, 1>{});
-  else if (MAX_PER == 2 || per == 2) fold(std::integral_constant<int, 2>{});
+  if (MAX_PER == 1 || per == 1) fold(std::integral_constant<int, 1>{});
+  else if (MAX_PER == 2 || per == 2) fold(std::integral_constant<int, MAX_PER < 2 ? MAX_PER : 2>{});
   else if (per <= 4) fold(std::integral_constant<int, MAX_PER < 4 ? MAX_PER : 4>{});
   else fold(std::integral_constant<int, MAX_PER>{});
 }
@@ -1383,12 +1387,12 @@ __device__ __forceinline__ Pack<V, AGG> block_total(Pack<V, AGG> share) {
   return total;
 }
 
-// `count` partial vectors added by the block in a fixed order, BLOCK * 4 loads at a time; valid in every thread.
-template <class G, int BLOCK, bool FINISH>
+// `count` partial vectors added by the block in a fixed order, BLOCK * BATCH loads at a time; valid in every thread.
+template <class G, int BLOCK, bool FINISH, int BATCH = 4>
 __device__ __forceinline__ Pack<typename G::Value, G::AGG_WIDTH>
 sum_partials(const typename G::Value* __restrict__ partials, const int count) {
   using V = typename G::Value;
-  constexpr int AGG = G::AGG_WIDTH, BATCH = 4;
+  constexpr int AGG = G::AGG_WIDTH;
   Pack<V, AGG> acc;
   zero(acc);
   for (int j0 = threadIdx.x; j0 < count; j0 += BATCH * BLOCK) {
@@ -1440,7 +1444,8 @@ __device__ __forceinline__ bool last_block(unsigned* counters, const int block, 
   return true;
 }
 
-template <class G, int BLOCK, int PARTS_PER_TILE>
+// SUM_BLOCK: block 0 adds up the aggregators' partials, the others fold the carries of BLOCK tiles each.
+template <class G, int BLOCK, int PARTS_PER_TILE, bool SUM_BLOCK>
 __global__ void __launch_bounds__(BLOCK)
 fixup_kernel(const int* __restrict__ carry_row, const typename G::Value* __restrict__ agg_partials,
              const typename G::Value* __restrict__ carry_val, const int num_tiles, const int per,
@@ -1448,8 +1453,19 @@ fixup_kernel(const int* __restrict__ carry_row, const typename G::Value* __restr
   using V = typename G::Value;
   constexpr int AGG = G::AGG_WIDTH;
   Pack<V, AGG> acc;
-  fixup_tiles<G, BLOCK, PARTS_PER_TILE, 8, false>(p, (int)blockIdx.x, num_tiles, per, carry_row, carry_val, agg_partials, acc);
-  if constexpr (AGG > 0) {
+  if constexpr (SUM_BLOCK) {
+    if (blockIdx.x == 0) {
+      const Pack<V, AGG> all = sum_partials<G, BLOCK, false, 8>(agg_partials, num_tiles * PARTS_PER_TILE);
+      if (threadIdx.x == 0) G::store_agg(p, all);
+    } else {
+      fixup_tiles<G, BLOCK, PARTS_PER_TILE, 1, false, false>(p, (int)blockIdx.x - 1, num_tiles, 1, carry_row, carry_val,
+                                                             agg_partials, acc);
+    }
+    return;
+  }
+  fixup_tiles<G, BLOCK, PARTS_PER_TILE, 4, false, true>(p, (int)blockIdx.x, num_tiles, per, carry_row, carry_val,
+                                                        agg_partials, acc);
+  if constexpr (AGG > 0 && !SUM_BLOCK) {
     __shared__ int s_is_last;
     const Pack<V, AGG> total = block_total<V, AGG, BLOCK>(acc);
     if (gridDim.x == 1) {
@@ -1516,7 +1532,7 @@ reduce_kernel(int2* coords, int* splits, const int* __restrict__ row_end, const 
       if (!last_block(counters, tile, tl.num_tiles, arrival)) return;
       constexpr int AGG = G::AGG_WIDTH;
       Pack<typename G::Value, AGG> acc;
-      fixup_tiles<G, BLOCK, partials_per_tile<BLOCK>(), (EARLY ? 4 : 2), true>(p, 0, tl.num_tiles, (tl.num_tiles + BLOCK - 1) / BLOCK,
+      fixup_tiles<G, BLOCK, partials_per_tile<BLOCK>(), (EARLY ? 4 : 2), true, true>(p, 0, tl.num_tiles, (tl.num_tiles + BLOCK - 1) / BLOCK,
                                                                          carry_row, carry_val, agg_partials, acc);
       if constexpr (AGG > 0) {
         const Pack<typename G::Value, AGG> total = block_total<typename G::Value, AGG, BLOCK>(acc);

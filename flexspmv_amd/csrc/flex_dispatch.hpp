@@ -156,9 +156,9 @@ inline int resident_grid(KernelT kernel, int block_threads, GridCache& cache) {
 #define FLEX_TUNE_INBLOCK_MAX_TILES 4096  // launches of at most this many tiles search inside the reducer blocks
 #endif
 #ifndef FLEX_TUNE_SINGLE_FIXUP_MAX_TILES
-#define FLEX_TUNE_SINGLE_FIXUP_MAX_TILES 4096  // launches of at most this many tiles fold carries and aggregators in one block
+#define FLEX_TUNE_SINGLE_FIXUP_MAX_TILES 8192  // launches of at most this many tiles add up their aggregators in one block
 #endif
-constexpr int SINGLE_FIXUP_BLOCK = 1024;
+constexpr int SUM_FIXUP_BLOCK = 1024;
 // A launch with counters (flexspmv_launch_args.counters) finishes itself, without a second kernel, up to 512 tiles of
 // 4-byte values or 256 of 8-byte values.  Such a launch runs for less than the 8 us it takes the host to issue two
 // kernels (2.7 to 4 us each): 256 x 256 Laplacian float32, 192 tiles, 8.2 -> 5.9 us a pass.  On the GPU the second kernel
@@ -168,6 +168,10 @@ constexpr int SINGLE_FIXUP_BLOCK = 1024;
 // such launches finish themselves up to 1 024 tiles.
 // (512 x 512 points, 1 024 tiles: float32 8.2 -> 7.3 us, float64 9.3 -> 8.4 against two kernels; with the 8 tiles a thread that
 // 2 000 tiles would need, the kernel's registers cost it a block per CU.)
+// Where there is no aggregator and tiles start anywhere, almost every tile leaves a record, and the last block's fold is a
+// longer way than a kernel of several blocks as soon as there are a few groups of them: 12 000 rows of 20 to 50 entries
+// (210 tiles of float32) 7.9 us in one kernel, 7.3 in two, 8 000 rows (140) 7.5 and 7.5, R-MAT scale 12 (26) 7.1 and 7.6.
+constexpr int FINISH_CARRY_MAX_TILES = 128;
 constexpr int FINISH_MAX_TILES = FIXUP_BLOCK * 2;
 constexpr int FINISH_EARLY_MAX_TILES = FIXUP_BLOCK * 4;
 template <typename V> constexpr int finish_max_tiles() { return FINISH_MAX_TILES * 4 / (int)sizeof(V); }
@@ -194,9 +198,9 @@ struct Dispatch {
     int num_tiles;
     int flat_blocks;
     bool search_in_blocks;
-    bool single_fixup;
     bool can_finish;                          // the reducer's last block can do the fix-up
-    int fixup_block, fixup_per, fixup_blocks;  // threads of a fixup_kernel block, tiles per thread, blocks
+    bool sum_block;                           // fixup_kernel: one more block, which adds up the aggregators
+    int fixup_block, fixup_per, fixup_blocks;  // ... threads of a block, tiles per thread, blocks that fold carries
     size_t off_coords, off_splits, off_carry_row, off_carry_val, off_partials, off_block_partials, off_ticket, total;
   };
 
@@ -263,10 +267,6 @@ struct Dispatch {
     l.num_tiles = l.tiling.num_tiles;
     l.flat_blocks = l.num_tiles < MAX_PERSISTENT_BLOCKS ? l.num_tiles : MAX_PERSISTENT_BLOCKS;
     l.search_in_blocks = REDUCER && l.num_tiles <= FLEX_TUNE_INBLOCK_MAX_TILES;
-    // ... twice as many where tiles start on rows: hardly a tile carries then, and the block only walks the records
-    // (spring-mass 100^3, 4 606 tiles: 2.6 us; with a carry per tile 8 192 tiles cost one block 20 us)
-    l.single_fixup = REDUCER && l.num_tiles <= FLEX_TUNE_SINGLE_FIXUP_MAX_TILES * (l.tiling.snap_slack > 0 ? 2 : 1) &&
-                     l.num_tiles <= 8 * SINGLE_FIXUP_BLOCK;
     size_t off = 0;
     l.off_coords = off;
     if (REDUCER) off += align_up(sizeof(int2) * ((size_t)l.num_tiles + 1));
@@ -276,14 +276,17 @@ struct Dispatch {
     if (REDUCER) off += align_up(sizeof(int) * (size_t)l.num_tiles);
     l.off_carry_val = off;
     if (REDUCER) off += align_up(sizeof(V) * (size_t)l.num_tiles * (G::RED_WIDTH > 0 ? G::RED_WIDTH : 1));
-    // (fixup_kernel: one block takes up to 8 tiles per thread; several blocks one, or eight where tiles hardly carry)
     // A launch small enough to finish itself is folded by 256 threads either way: the same sums in the same order.
-    const bool early = G::AGG_WIDTH == 0 && l.tiling.snap_slack > 0;
-    const bool small = l.single_fixup && l.num_tiles <= (early ? FINISH_EARLY_MAX_TILES : FINISH_MAX_TILES);
-    l.fixup_block = l.single_fixup && !small ? SINGLE_FIXUP_BLOCK : FIXUP_BLOCK;
-    if (l.single_fixup) l.fixup_per = (l.num_tiles + l.fixup_block - 1) / l.fixup_block;
-    else l.fixup_per = l.tiling.snap_slack > 0 ? 8 : 1;
-    l.can_finish = small && (early || l.num_tiles <= finish_max_tiles<V>()) && BLOCK == FIXUP_BLOCK;
+    const bool snapped = l.tiling.snap_slack > 0;
+    const int finish_tiles = G::AGG_WIDTH > 0 ? finish_max_tiles<V>() : snapped ? FINISH_EARLY_MAX_TILES : FINISH_CARRY_MAX_TILES;
+    const bool small = l.num_tiles <= (G::AGG_WIDTH > 0 ? FINISH_MAX_TILES : finish_tiles) &&
+                       l.num_tiles <= FLEX_TUNE_SINGLE_FIXUP_MAX_TILES;
+    l.can_finish = small && l.num_tiles <= finish_tiles && BLOCK == FIXUP_BLOCK;
+    l.sum_block = G::AGG_WIDTH > 0 && !small && l.num_tiles <= FLEX_TUNE_SINGLE_FIXUP_MAX_TILES;
+    l.fixup_block = l.sum_block ? SUM_FIXUP_BLOCK : FIXUP_BLOCK;
+    // Two tiles a thread where tiles hardly carry and every block draws a ticket: half as many tickets (y = A x, y . x on
+    // 250^3 points float64 290.7 us, 292.2 with one, 290.4 with eight; R-MAT scale 21 with int64 sums 194.1, 193.9, 197.2).
+    l.fixup_per = small ? (l.num_tiles + l.fixup_block - 1) / l.fixup_block : G::AGG_WIDTH > 0 && snapped && !l.sum_block ? 2 : 1;
     const int per_block = l.fixup_block * l.fixup_per;
     l.fixup_blocks = (l.num_tiles + per_block - 1) / per_block;
     l.off_partials = off;
@@ -448,12 +451,17 @@ struct Dispatch {
         V* block_partials = (V*)(ws + l.off_block_partials);
         constexpr int PARTS = partials_per_tile<BLOCK>();
         auto launch_fixup = [&](auto kernel) {
-          hipLaunchKernelGGL(kernel, dim3(l.fixup_blocks), dim3(l.fixup_block), 0, stream, (const int*)carry_row,
+          const int blocks = l.fixup_blocks + (l.sum_block ? 1 : 0);
+          hipLaunchKernelGGL(kernel, dim3(blocks), dim3(l.fixup_block), 0, stream, (const int*)carry_row,
                              (const V*)partials, (const V*)carry_val, l.num_tiles, l.fixup_per, block_partials, ticket, p);
-          report(l.single_fixup ? "fixup_kernel (one block)" : "fixup_kernel", kernel, l.fixup_blocks, l.fixup_block);
+          report(blocks == 1 ? "fixup_kernel (one block)" : "fixup_kernel", kernel, blocks, l.fixup_block);
         };
-        if (l.fixup_block == SINGLE_FIXUP_BLOCK) launch_fixup(fixup_kernel<G, SINGLE_FIXUP_BLOCK, PARTS>);
-        else launch_fixup(fixup_kernel<G, FIXUP_BLOCK, PARTS>);
+        if constexpr (G::AGG_WIDTH > 0) {
+          if (l.sum_block) launch_fixup(fixup_kernel<G, SUM_FIXUP_BLOCK, PARTS, true>);
+          else launch_fixup(fixup_kernel<G, FIXUP_BLOCK, PARTS, false>);
+        } else {
+          launch_fixup(fixup_kernel<G, FIXUP_BLOCK, PARTS, false>);
+        }
       }
     } else {
       // edges per thread: as few as make at most FLAT_SMALL_BLOCKS blocks, at most IPT

@@ -11,8 +11,9 @@ from flexspmv_amd.binding import DTYPE_CODES, load_named
 
 pytestmark = pytest.mark.gpu
 
-# one tile; one, two, four and eight tiles per thread of the single block, and one more than each; the most tiles of
-# one block and one more (five blocks then, the last ticket adds their aggregator sums)
+# one tile and two (one block folds and adds up); around the blocks of 1 024 tiles that fold carries beside the block
+# that adds up, one to eight of them; the most tiles of that shape and one more (17 blocks of 512 tiles then, the last
+# ticket adds their aggregator sums)
 TILES = (1, 2, 1023, 1024, 1025, 2048, 2049, 4097, 8192, 8193, 12_300)
 
 
@@ -53,3 +54,33 @@ def test_integer_sums_at_every_fixup_shape(tiles):
         y, total = ext.merged_spmv_launch(w, ids, col, ptr, n, n)
         assert torch.equal(y, want_y)
         assert int(total) == int(want.sum())
+
+
+# Without an aggregator: the reducer's last block up to 128 tiles, blocks of 256 tiles from there on
+@pytest.mark.parametrize("tiles", (1, 2, 127, 128, 129, 256, 257, 513, 1024, 1025, 4097))
+def test_carries_without_an_aggregator(tiles):
+    ext = load_named("csr_spmv", build_if_missing=False)
+    out = (ctypes.c_int32 * 6)()
+    length = torch.full((max(2, tiles * 41),), 50, dtype=torch.int64)     # hardly a tile starts on a row of 50 entries
+    length[tiles // 2] = 20 * 2048 if tiles > 30 else 50                  # ... and a row of 20 tiles
+    ends = torch.cumsum(length, 0)
+    lo, hi = 1, ends.numel()
+    while lo < hi:                      # the fewest rows that make at least this many tiles
+        mid = (lo + hi) // 2
+        assert ext._lib.flexspmv_tiling(DTYPE_CODES["float32"], mid, int(ends[mid - 1]), out) == 0
+        lo, hi = (lo, mid) if out[0] >= tiles else (mid + 1, hi)
+    n, ne = lo, int(ends[lo - 1])
+    print(f"case carries {tiles} tiles {n} rows {ne} edges", flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(tiles)
+    ptr = torch.zeros(n + 1, dtype=torch.int32, device="cuda")
+    ptr[1:] = ends[:n].cuda()
+    col = torch.randint(0, n, (ne,), generator=gen, device="cuda", dtype=torch.int32)
+    rows = torch.repeat_interleave(torch.arange(n), length[:n]).cuda()
+    for dtype, top in ((torch.float32, 8), (torch.float64, 1 << 20)):
+        # whole numbers whose sums the type holds exactly: one right answer in every order
+        a = torch.randint(-top, top, (ne,), generator=gen, device="cuda").to(dtype)
+        x = torch.randint(-top, top, (n,), generator=gen, device="cuda").to(dtype)
+        (y,) = ext.merged_spmv_launch(a, x, col, ptr, n, n)
+        (again,) = ext._launch_checked((a, x, col, ptr, n, n), {})
+        want = torch.zeros(n, dtype=torch.float64, device="cuda").index_add_(0, rows, a.double() * x.double()[col.long()])
+        assert torch.equal(y.double(), want) and torch.equal(again, y)
