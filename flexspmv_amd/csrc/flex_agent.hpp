@@ -1097,13 +1097,13 @@ reduce_tile(const int tile, const int2 c0, const int2 c1, const Tiling& tl, cons
 // Small launches (flex_dispatch.hpp says which) are folded by 256 threads: the reducer's last block, or a kernel of one
 // block.  Larger ones use blocks of 256 threads with a tile per thread: where tiles carry, one block with several tiles a
 // thread spends longer on its runs than blocks side by side.
-// Aggregators up to 8 192 tiles: one more block, which only adds up the partials, beside blocks of 1 024 threads that
-// only fold carries, so that none waits for another.  Beyond, the block that draws the last ticket adds the blocks' sums,
+// Aggregators up to 8 192 tiles: one more block, which only adds up the partials, beside blocks that only fold carries,
+// so that none waits for another.  Beyond, the block that draws the last ticket adds the blocks' sums,
 // in block order.  What it reads was stored write-through at device scope and had arrived before the ticket was drawn, so
 // no block has to write its XCD's L2 back: that release cost 15 us a launch, a kernel of its own for the sum 4.7.
 // Per pass, one block of 1 024 threads up to 4 096 tiles (8 192 row-snapped ones) -> this: 200 000 rows of 20 to 50
-// entries, float32 31.2 -> 18.0 us; R-MAT scale 19 float32 44.4 -> 34.1, float64 63.6 -> 50.7, int64 sums 67.1 -> 53.9;
-// spring-mass 100^3 24.3 -> 23.3.
+// entries, float32 31.2 -> 18.0 us; R-MAT scale 19 float32 44.4 -> 34.1, float64 63.6 -> 50.7, int64 sums 67.1 -> 53.9,
+// scale 16 12.9 -> 11.9; spring-mass 100^3 24.3 -> 23.3.
 // ----------------------------------------------------------------------------------------------
 
 // Tiles [first, first + BLOCK * PER).  acc: receives the thread's share of the aggregators.
@@ -1455,6 +1455,7 @@ fixup_kernel(const int* __restrict__ carry_row, const typename G::Value* __restr
   Pack<V, AGG> acc;
   if constexpr (SUM_BLOCK) {
     if (blockIdx.x == 0) {
+      // (8: 256 threads take 2 048 partials at once, 1 024 threads 8 192)
       const Pack<V, AGG> all = sum_partials<G, BLOCK, false, 8>(agg_partials, num_tiles * PARTS_PER_TILE);
       if (threadIdx.x == 0) G::store_agg(p, all);
     } else {

@@ -158,7 +158,12 @@ inline int resident_grid(KernelT kernel, int block_threads, GridCache& cache) {
 #ifndef FLEX_TUNE_SINGLE_FIXUP_MAX_TILES
 #define FLEX_TUNE_SINGLE_FIXUP_MAX_TILES 8192  // launches of at most this many tiles add up their aggregators in one block
 #endif
+// Threads of a block of such a launch's fix-up: 256 up to 2 048 tiles, where more blocks that fold fewer carries each pay
+// (R-MAT scale 16 and 17 with int64 sums 11.9 and 17.2 us; with 512 threads 12.4 and 17.5, with 1 024 12.9 and 18.3),
+// 1 024 beyond, where the block that adds up has more partials than 256 threads load at once (spring-mass 100^3, 4 606
+// tiles: float32 23.6, float64 45.1; with 256 threads 24.1 and 45.9).
 constexpr int SUM_FIXUP_BLOCK = 1024;
+constexpr int SUM_FIXUP_SMALL_TILES = 2048;
 // A launch with counters (flexspmv_launch_args.counters) finishes itself, without a second kernel, up to 512 tiles of
 // 4-byte values or 256 of 8-byte values.  Such a launch runs for less than the 8 us it takes the host to issue two
 // kernels (2.7 to 4 us each): 256 x 256 Laplacian float32, 192 tiles, 8.2 -> 5.9 us a pass.  On the GPU the second kernel
@@ -279,11 +284,10 @@ struct Dispatch {
     // A launch small enough to finish itself is folded by 256 threads either way: the same sums in the same order.
     const bool snapped = l.tiling.snap_slack > 0;
     const int finish_tiles = G::AGG_WIDTH > 0 ? finish_max_tiles<V>() : snapped ? FINISH_EARLY_MAX_TILES : FINISH_CARRY_MAX_TILES;
-    const bool small = l.num_tiles <= (G::AGG_WIDTH > 0 ? FINISH_MAX_TILES : finish_tiles) &&
-                       l.num_tiles <= FLEX_TUNE_SINGLE_FIXUP_MAX_TILES;
-    l.can_finish = small && l.num_tiles <= finish_tiles && BLOCK == FIXUP_BLOCK;
+    const bool small = l.num_tiles <= finish_tiles && l.num_tiles <= FLEX_TUNE_SINGLE_FIXUP_MAX_TILES;
+    l.can_finish = small && BLOCK == FIXUP_BLOCK;
     l.sum_block = G::AGG_WIDTH > 0 && !small && l.num_tiles <= FLEX_TUNE_SINGLE_FIXUP_MAX_TILES;
-    l.fixup_block = l.sum_block ? SUM_FIXUP_BLOCK : FIXUP_BLOCK;
+    l.fixup_block = l.sum_block && l.num_tiles > SUM_FIXUP_SMALL_TILES ? SUM_FIXUP_BLOCK : FIXUP_BLOCK;
     // Two tiles a thread where tiles hardly carry and every block draws a ticket: half as many tickets (y = A x, y . x on
     // 250^3 points float64 290.7 us, 292.2 with one, 290.4 with eight; R-MAT scale 21 with int64 sums 194.1, 193.9, 197.2).
     l.fixup_per = small ? (l.num_tiles + l.fixup_block - 1) / l.fixup_block : G::AGG_WIDTH > 0 && snapped && !l.sum_block ? 2 : 1;
@@ -457,7 +461,8 @@ struct Dispatch {
           report(blocks == 1 ? "fixup_kernel (one block)" : "fixup_kernel", kernel, blocks, l.fixup_block);
         };
         if constexpr (G::AGG_WIDTH > 0) {
-          if (l.sum_block) launch_fixup(fixup_kernel<G, SUM_FIXUP_BLOCK, PARTS, true>);
+          if (l.sum_block && l.fixup_block == SUM_FIXUP_BLOCK) launch_fixup(fixup_kernel<G, SUM_FIXUP_BLOCK, PARTS, true>);
+          else if (l.sum_block) launch_fixup(fixup_kernel<G, FIXUP_BLOCK, PARTS, true>);
           else launch_fixup(fixup_kernel<G, FIXUP_BLOCK, PARTS, false>);
         } else {
           launch_fixup(fixup_kernel<G, FIXUP_BLOCK, PARTS, false>);

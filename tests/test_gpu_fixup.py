@@ -11,9 +11,9 @@ from flexspmv_amd.binding import DTYPE_CODES, load_named
 
 pytestmark = pytest.mark.gpu
 
-# one tile and two (one block folds and adds up); around the blocks of 1 024 tiles that fold carries beside the block
-# that adds up, one to eight of them; the most tiles of that shape and one more (17 blocks of 512 tiles then, the last
-# ticket adds their aggregator sums)
+# one tile and two (one block folds and adds up); blocks of 256 tiles that fold carries beside the block that adds up,
+# four to eight of them; blocks of 1 024 tiles; the most tiles of that shape and one more (17 blocks of 512
+# tiles then, the last ticket adds their aggregator sums)
 TILES = (1, 2, 1023, 1024, 1025, 2048, 2049, 4097, 8192, 8193, 12_300)
 
 
@@ -84,3 +84,9 @@ def test_carries_without_an_aggregator(tiles):
         (again,) = ext._launch_checked((a, x, col, ptr, n, n), {})
         want = torch.zeros(n, dtype=torch.float64, device="cuda").index_add_(0, rows, a.double() * x.double()[col.long()])
         assert torch.equal(y.double(), want) and torch.equal(again, y)
+
+
+# With an aggregator: the reducer's last block up to 256 tiles of 8-byte values, then blocks that fold beside one that adds
+@pytest.mark.parametrize("tiles", (255, 256, 257, 511, 512, 513, 767))
+def test_integer_sums_around_the_smallest_launches(tiles):
+    test_integer_sums_at_every_fixup_shape(tiles)
