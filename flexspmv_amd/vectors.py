@@ -64,8 +64,9 @@ class ConjugateGradientUpdates:
         self._lib = library()
 
     def takes(self, ap, pap) -> bool:
-        return (ap.dtype == self._dtype and ap.device == self._device and ap.numel() == self._n and ap.is_contiguous()
-                and pap.dtype == self._dtype and pap.device == self._device and pap.numel() > 0)
+        return (ap.dtype == self._dtype and ap.device == self._device and ap.shape == (self._n,) and ap.is_contiguous()
+                and pap.dtype == self._dtype and pap.device == self._device and pap.dim() == 1 and pap.numel() > 0
+                and not ap.requires_grad and not pap.requires_grad)
 
     def step(self, x, r, p, ap, rr, pap) -> Tuple["torch.Tensor", "torch.Tensor"]:
         """Updates ``x`` and ``r`` in place; returns the next direction and the new ``r . r`` (0-dim, on the device)."""
