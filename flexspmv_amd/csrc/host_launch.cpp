@@ -12,7 +12,6 @@
 
 #include <ATen/core/Tensor.h>
 #include <ATen/hip/EmptyTensor.h>
-#include <ATen/ops/zeros.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime_api.h>
@@ -122,18 +121,26 @@ PyObject* scratch_of(Launcher* self, PyObject* ext, const c10::Device& device, l
 // Counters of launches on a stream of a device (flexspmv_launch_args.counters): cleared when they are made, left at zero
 // by every launch, shared by all libraries - launches on one stream are ordered.  Held under the GIL; made on the stream
 // they serve, so that the caching allocator hands a dropped block out again in that stream's order.  Never destroyed at
-// exit (the allocator may be gone by then).
+// exit (the allocator may be gone by then).  The caller keeps the tensor until its launch is issued: another thread may
+// drop all counters while this one issues without the GIL.
 constexpr size_t MAX_COUNTERS = 64;
-void* counters_of(const c10::Device& device, hipStream_t stream) {
-  if (stream == hipStreamPerThread) return nullptr;  // one handle for a stream per thread
+at::Tensor counters_of(const c10::Device& device, hipStream_t stream) {
+  if (stream == hipStreamPerThread) return at::Tensor();  // one handle for a stream per thread
   static auto* known = new std::map<std::pair<int, hipStream_t>, at::Tensor>();
   const auto key = std::make_pair((int)device.index(), stream);
   auto it = known->find(key);
   if (it == known->end()) {
     if (known->size() >= MAX_COUNTERS) known->clear();
-    it = known->emplace(key, at::zeros({FLEXSPMV_COUNTER_BYTES}, at::TensorOptions().dtype(at::kByte).device(device))).first;
+    // allocated and cleared past the dispatcher: under a mode that makes other tensors of it (fake ones) too
+    const int64_t size = FLEXSPMV_COUNTER_BYTES;
+    at::Tensor made(at::detail::empty_cuda(c10::IntArrayRef(&size, 1), at::kByte, device, std::nullopt));
+    if (hipMemsetAsync(made.data_ptr(), 0, (size_t)size, stream) != hipSuccess) {
+      (void)hipGetLastError();
+      return at::Tensor();
+    }
+    it = known->emplace(key, std::move(made)).first;
   }
-  return it->second.data_ptr();
+  return it->second;
 }
 
 constexpr int MAX_POINTERS = 64;  // of one kind; a library with more goes through Python
@@ -241,7 +248,8 @@ PyObject* launcher_launch(PyObject* self_obj, PyObject* const* call, Py_ssize_t 
   la.workspace = ws.data_ptr();
   la.workspace_bytes = (size_t)ws.numel();
   la.stream = stream;
-  la.counters = counters_of(device, stream);
+  const at::Tensor counters = counters_of(device, stream);
+  la.counters = counters.defined() ? counters.data_ptr() : nullptr;
   int rc;
   {
     pybind11::gil_scoped_release no_gil;

@@ -112,3 +112,31 @@ def test_blocks_arrive_early(n, kind):
             exact = torch.zeros(n, dtype=torch.float64, device="cuda").index_add_(0, rows, a.double() * x.double()[col.long()])
             # every term positive: at most a rounding per term of the longest row
             assert bool(((want.double() - exact).abs() <= int(lengths.max()) * torch.finfo(dtype).eps * exact).all())
+
+
+def test_more_streams_than_counters_are_kept_for():
+    """Counters are kept for 64 streams; with more they are dropped and made again, and stay at zero."""
+    import ctypes
+    with open("/proc/self/maps") as maps:         # the runtime that torch has loaded, not a second one
+        hip = ctypes.CDLL(next(line.split()[-1] for line in maps if "libamdhip64" in line))
+    streams = []
+    for _ in range(70):
+        handle = ctypes.c_void_p()
+        assert hip.hipStreamCreate(ctypes.byref(handle)) == 0
+        streams.append(torch.cuda.ExternalStream(handle.value))
+    n = 20_000
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    ptr = torch.arange(0, 4 * n + 1, 4, dtype=torch.int32, device="cuda")
+    col = torch.randint(0, n, (4 * n,), generator=gen, device="cuda", dtype=torch.int32)
+    rows = torch.arange(n, dtype=torch.int32, device="cuda").repeat_interleave(4)
+    ext = load_named("spmv_dot", build_if_missing=False)
+    args = (torch.rand(4 * n, generator=gen, device="cuda"), torch.rand(n, generator=gen, device="cuda"), col, rows, ptr, n, n)
+    want = ext._launch_checked(args, {})
+    torch.cuda.synchronize()
+    for _ in range(2):
+        for k, stream in enumerate(streams):
+            print(f"case counters of stream {k}", flush=True)
+            with torch.cuda.stream(stream):
+                got = ext.merged_spmv_launch(*args)
+            stream.synchronize()
+            assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
