@@ -144,9 +144,10 @@ rows_search_kernel(const I* __restrict__ rows, const int ne, const int num_rows,
 
 // ---------------------------------------------------------------------------------------------------
 // Stable sort of (row id, position) pairs: least-significant-digit radix sort, 8-bit digits over the
-// bits num_rows needs.  Three kernels per digit, no atomics on memory and nothing to clear beforehand:
-//   sort_histogram_kernel   block b counts the digits of its chunk of tiles -> hist[digit][b]
-//   sort_scan_kernel        block d turns row d of hist into exclusive prefixes and leaves the row's sum
+// bits num_rows needs.  Three kernels per digit (two for short lists), no atomics on memory and nothing to clear beforehand:
+//   sort_histogram_kernel   block b counts the digits of its chunk of tiles -> hist[digit][b] (short lists: [b][digit])
+//   sort_scan_kernel        block d turns row d of hist into exclusive prefixes and leaves the row's sum (short lists:
+//                           none, the scatter adds up for itself)
 //   sort_scatter_kernel     block b ranks its tiles' items (wave64 ballots give every item the lanes that
 //                           hold the same digit; wavefront counters in LDS carry the order across the 16
 //                           items of a lane and across the block's wavefronts), orders a tile by digit in LDS
@@ -179,6 +180,11 @@ constexpr long long BIG_SCATTER_FROM = 16ll << 20;   // pairs
 constexpr int SORT_MAX_BLOCKS = 4096;                   // a block takes several tiles beyond that many
 constexpr int SORT_SCAN_ITEMS = SORT_MAX_BLOCKS / BLOCK;
 constexpr int SORT_MAX_PASSES = 4;
+// Up to this many blocks the scatter's blocks add up the counts of all blocks for themselves instead of waiting for a
+// kernel that scans them: a digit is two launches then, and a launch of a dependent chain costs more than the sums as
+// long as these are few.  Two digits, us per sort with the kernel and without: 5 blocks (20 000 pairs) 29.5, 24.6;
+// 25 blocks 29.3, 25.1; 49 blocks 31.1, 29.0; 64 blocks 30.4, 28.5; 98 blocks 32.2, 33.1; 128 blocks 33.5, 35.8.
+constexpr int SORT_OWN_SCAN_BLOCKS = 64;
 static_assert(RADIX == BLOCK && BIG_SCATTER_BLOCK % BLOCK == 0, "thread d < 256 of a block owns digit d");
 
 // Ids outside [0, num_rows) sort as the last row, num_rows - 1 (a digit more for them would cost a whole
@@ -226,7 +232,8 @@ __device__ inline unsigned block_exclusive_sum(const unsigned v, unsigned* s_tmp
 template <typename I, bool FIRST>
 __global__ void __launch_bounds__(BLOCK)
 sort_histogram_kernel(const void* __restrict__ keys_in, const long long ne, const unsigned last_row, const int shift,
-                      const unsigned mask, const int tiles_per_block, const int blocks, unsigned* __restrict__ hist) {
+                      const unsigned mask, const int tiles_per_block, const int digit_stride, const int block_stride,
+                      unsigned* __restrict__ hist) {
   __shared__ unsigned s_cnt[SORT_WAVES][RADIX];
   const int lane = threadIdx.x & (WAVE - 1), wave = threadIdx.x / WAVE;
 #pragma unroll
@@ -261,7 +268,7 @@ sort_histogram_kernel(const void* __restrict__ keys_in, const long long ne, cons
   unsigned sum = 0;
 #pragma unroll
   for (int w = 0; w < SORT_WAVES; ++w) sum += s_cnt[w][threadIdx.x];
-  hist[(size_t)threadIdx.x * blocks + blockIdx.x] = sum;
+  hist[(size_t)threadIdx.x * digit_stride + (size_t)blockIdx.x * block_stride] = sum;
 }
 
 __global__ void __launch_bounds__(BLOCK)
@@ -412,7 +419,8 @@ __device__ inline void scatter_tile(ScatterShared<THREADS>& sh, const void* __re
 
 // BITS: how many bits the digits of this pass have at most - the ranking takes six vector instructions per bit and item
 // (20 M pairs, 3 M rows, digits of 8, 7 and 7 bits: the passes of 7 bits 110.0 -> 107.5 us each, ranked by 8 bits before).
-template <typename I, bool FIRST, int THREADS, int BITS>
+// SCANNED: hist and totals are sort_scan_kernel's; else hist holds the counts themselves, digits next to each other.
+template <typename I, bool FIRST, int THREADS, int BITS, bool SCANNED>
 __global__ void __launch_bounds__(THREADS)
 sort_scatter_kernel(const void* __restrict__ keys_in, const int32_t* __restrict__ vals_in,
                     unsigned* __restrict__ keys_out, int32_t* __restrict__ vals_out, const long long ne,
@@ -423,8 +431,26 @@ sort_scatter_kernel(const void* __restrict__ keys_in, const int32_t* __restrict_
   const int t = threadIdx.x;
   // thread t follows digit t: the digit's place in the output, then this block's place among the blocks
   unsigned unused;
-  unsigned next_of_digit = block_exclusive_sum<THREADS / WAVE>(t < RADIX ? totals[t] : 0u, sh.tmp, unused);
-  if (t < RADIX) next_of_digit += hist[(size_t)t * blocks + blockIdx.x];
+  unsigned next_of_digit;
+  if constexpr (SCANNED) {
+    next_of_digit = block_exclusive_sum<THREADS / WAVE>(t < RADIX ? totals[t] : 0u, sh.tmp, unused);
+    if (t < RADIX) next_of_digit += hist[(size_t)t * blocks + blockIdx.x];
+  } else {
+    static_assert(THREADS == RADIX, "a thread per digit");
+    unsigned before = 0, total = 0;
+    constexpr int STEP = 16;   // counts in flight per thread
+    for (int j = 0; j < blocks; j += STEP) {
+      unsigned c[STEP];
+#pragma unroll
+      for (int u = 0; u < STEP; ++u) c[u] = hist[(size_t)min(j + u, blocks - 1) * RADIX + t];
+#pragma unroll
+      for (int u = 0; u < STEP; ++u) {
+        if (j + u < blocks) total += c[u];
+        if (j + u < (int)blockIdx.x) before += c[u];
+      }
+    }
+    next_of_digit = block_exclusive_sum<THREADS / WAVE>(total, sh.tmp, unused) + before;
+  }
   const long long first_tile = (long long)blockIdx.x * tiles_per_block;
   for (int tl = 0; tl < tiles_per_block; ++tl) {
     const long long tile_at = (first_tile + tl) * TILE;
@@ -494,34 +520,37 @@ hipError_t sort_pairs(const SortPlan& p, void* workspace, const I* rows, int32_t
     const unsigned last_row = (unsigned)(num_rows - 1);
     // a block of the histogram counts the pairs the scatter's block of the same number moves
     const int count_tiles = p.tiles_per_block * (p.scatter_threads * SORT_ITEMS / COUNT_TILE);
+    const bool scanned = p.blocks > SORT_OWN_SCAN_BLOCKS || p.scatter_threads != BLOCK;
+    const int digit_stride = scanned ? p.blocks : 1, block_stride = scanned ? 1 : RADIX;
     if (i == 0) {
       hipLaunchKernelGGL((sort_histogram_kernel<I, true>), grid, block, 0, stream, keys_in, (long long)ne, last_row,
-                         p.shift[i], mask, count_tiles, p.blocks, hist);
+                         p.shift[i], mask, count_tiles, digit_stride, block_stride, hist);
     } else {
       hipLaunchKernelGGL((sort_histogram_kernel<int32_t, false>), grid, block, 0, stream, keys_in, (long long)ne,
-                         last_row, p.shift[i], mask, count_tiles, p.blocks, hist);
+                         last_row, p.shift[i], mask, count_tiles, digit_stride, block_stride, hist);
     }
-    hipLaunchKernelGGL(sort_scan_kernel, dim3(RADIX), block, 0, stream, hist, p.blocks, totals);
-    auto scatter = [&](auto first, auto threads, auto bits) {
-      constexpr bool FIRST = decltype(first)::value;
+    if (scanned) hipLaunchKernelGGL(sort_scan_kernel, dim3(RADIX), block, 0, stream, hist, p.blocks, totals);
+    auto scatter = [&](auto first, auto threads, auto own_scan, auto bits) {
+      constexpr bool FIRST = decltype(first)::value, SCANNED = !decltype(own_scan)::value;
       constexpr int THREADS = decltype(threads)::value;
       using Id = typename std::conditional<FIRST, I, int32_t>::type;
-      hipLaunchKernelGGL((sort_scatter_kernel<Id, FIRST, THREADS, decltype(bits)::value>), grid, dim3(THREADS), 0, stream,
-                         keys_in, vals_in, keys_out, vals_out, (long long)ne, last_row, p.shift[i], mask,
+      hipLaunchKernelGGL((sort_scatter_kernel<Id, FIRST, THREADS, decltype(bits)::value, SCANNED>), grid, dim3(THREADS), 0,
+                         stream, keys_in, vals_in, keys_out, vals_out, (long long)ne, last_row, p.shift[i], mask,
                          p.tiles_per_block, p.blocks, (const unsigned*)hist, (const unsigned*)totals);
     };
-    auto scatter_of = [&](auto first, auto threads) {
-      if (p.bits[i] <= 6) scatter(first, threads, std::integral_constant<int, 6>{});
-      else if (p.bits[i] == 7) scatter(first, threads, std::integral_constant<int, 7>{});
-      else scatter(first, threads, std::integral_constant<int, RADIX_BITS>{});
+    auto scatter_of = [&](auto threads, auto own_scan) {
+      auto with_bits = [&](auto first) {
+        if (p.bits[i] <= 6) scatter(first, threads, own_scan, std::integral_constant<int, 6>{});
+        else if (p.bits[i] == 7) scatter(first, threads, own_scan, std::integral_constant<int, 7>{});
+        else scatter(first, threads, own_scan, std::integral_constant<int, RADIX_BITS>{});
+      };
+      if (i == 0) with_bits(std::true_type{}); else with_bits(std::false_type{});
     };
     using Big = std::integral_constant<int, BIG_SCATTER_BLOCK>;
     using Small = std::integral_constant<int, BLOCK>;
-    if (p.scatter_threads == BIG_SCATTER_BLOCK) {
-      if (i == 0) scatter_of(std::true_type{}, Big{}); else scatter_of(std::false_type{}, Big{});
-    } else {
-      if (i == 0) scatter_of(std::true_type{}, Small{}); else scatter_of(std::false_type{}, Small{});
-    }
+    if (!scanned) scatter_of(Small{}, std::true_type{});
+    else if (p.scatter_threads == BIG_SCATTER_BLOCK) scatter_of(Big{}, std::false_type{});
+    else scatter_of(Small{}, std::false_type{});
     keys_in = keys_out;
     vals_in = vals_out;
   }
